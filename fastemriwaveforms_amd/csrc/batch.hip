@@ -6,6 +6,7 @@
 
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <vector>
 
@@ -87,7 +88,7 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
     std::map<std::pair<int, int>, int> rowmap;
     for (int r = 0; r < u.Nr; r++) rowmap[{u.row_m[r], u.row_k[r]}] = r;
     const int ncell = u.Nr * u.Nc;
-    std::vector<int> cells, ents;
+    std::vector<int> cells, ents, dstart, dmember, dcell(ncell);
     std::vector<long> sys_prefix(B + 1, 0);
     std::vector<int> seg_prefix(B + 1, 0);
     WaveDesc d{};
@@ -128,6 +129,32 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
             e[fill[cell_of(m[q], k[q], n[q])]++] = 2 * q;
             if (m[q] != 0) e[fill[cell_of(-m[q], -k[q], -n[q])]++] = 2 * q + 1;
         }
+        // cells of the FP64 direct sum: the distinct (m, k, n) in the order of
+        // their first modes, members ascending (the order of launch_cell_index)
+        std::fill(dcell.begin(), dcell.end(), -1);
+        std::vector<int> dsize, did(K);
+        for (int q = 0; q < K; q++) {
+            int &id = dcell[cell_of(m[q], k[q], n[q])];
+            if (id < 0) {
+                id = (int)dsize.size();
+                dsize.push_back(0);
+            }
+            dsize[id]++;
+            did[q] = id;
+        }
+        d.dcell_off = (int)dstart.size();
+        dstart.push_back((int)dsize.size());
+        int at = 0;
+        for (int &sz : dsize) {
+            dstart.push_back(at);
+            const int n_in = sz;
+            sz = at;  // fill position
+            at += n_in;
+        }
+        dstart.push_back(at);
+        const size_t mbase = dmember.size();
+        dmember.resize(mbase + K);
+        for (int q = 0; q < K; q++) dmember[mbase + dsize[did[q]]++] = q;
         cells.insert(cells.end(), cs.begin(), cs.end());
         ents.insert(ents.end(), e.begin(), e.end());
         bp->desc.push_back(d);
@@ -144,7 +171,7 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
         bp->total_intervals += L - 1;
         bp->total_tpref += L;
         bp->total_systems += 2L * K + 3;
-        bp->direct_blocks += ((long)N + 511) / 512 + (L - 1);
+        bp->direct_blocks += ((long)N + DIRECT_TILE - 1) / DIRECT_TILE + (L - 1);
         bp->fact16_blocks += ((long)N + 255) / 256 + (L - 1);
         mode_off += K;
     }
@@ -153,7 +180,8 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
     if (cells.empty()) cells.push_back(0);
     if (ents.empty()) ents.push_back(0);
 
-    // one device allocation: desc | sys_prefix | seg_prefix | row_mk | cells | ents | m | k | n
+    // one device allocation: desc | sys_prefix | seg_prefix | row_mk | cells | ents | m | k | n |
+    // the direct sum's cells
     size_t off = 0;
     const size_t o_desc = off; off = al256(off + sizeof(WaveDesc) * B);
     const size_t o_sys = off; off = al256(off + sizeof(long) * (B + 1));
@@ -164,6 +192,8 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
     const size_t o_m = off; off = al256(off + sizeof(int) * Ksum);
     const size_t o_k = off; off = al256(off + sizeof(int) * Ksum);
     const size_t o_n = off; off = al256(off + sizeof(int) * Ksum);
+    const size_t o_ds = off; off = al256(off + sizeof(int) * dstart.size());
+    const size_t o_dm = off; off = al256(off + sizeof(int) * dmember.size());
     std::vector<unsigned char> host(off, 0);
     memcpy(&host[o_desc], bp->desc.data(), sizeof(WaveDesc) * B);
     memcpy(&host[o_sys], sys_prefix.data(), sizeof(long) * (B + 1));
@@ -179,6 +209,8 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
     memcpy(&host[o_m], h_m, sizeof(int) * Ksum);
     memcpy(&host[o_k], h_k, sizeof(int) * Ksum);
     memcpy(&host[o_n], h_n, sizeof(int) * Ksum);
+    memcpy(&host[o_ds], dstart.data(), sizeof(int) * dstart.size());
+    memcpy(&host[o_dm], dmember.data(), sizeof(int) * dmember.size());
     if (hipGetDevice(&bp->device) != hipSuccess || hipMalloc(&bp->dev_buf, off) != hipSuccess ||
         hipMemcpy(bp->dev_buf, host.data(), off, hipMemcpyHostToDevice) != hipSuccess) {
         set_error("batch_create: device upload of %zu bytes failed", off);
@@ -199,6 +231,8 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
     D.m = reinterpret_cast<const int *>(base + o_m);
     D.k = reinterpret_cast<const int *>(base + o_k);
     D.n = reinterpret_cast<const int *>(base + o_n);
+    D.dcell_start = reinterpret_cast<const int *>(base + o_ds);
+    D.dcell_member = reinterpret_cast<const int *>(base + o_dm);
     FactPlanDev &U = D.uni;
     U.K = 0;
     U.Nr = u.Nr;
@@ -295,7 +329,7 @@ int few_batch_run_async(const void *batch, const double *t, const double *teuk,
                   reinterpret_cast<int *>(w + L.wt), 0};
     BatchPtrs p{t, teuk, phase_knots, ylm, interp, pcoef, reinterpret_cast<double *>(w + L.region),
                 static_cast<double2 *>(wave)};
-    const int tile = precision == FEW_PRECISION_FP64 ? direct_tile(FEW_PRECISION_FP64)
+    const int tile = precision == FEW_PRECISION_FP64 ? DIRECT_TILE
                                                      : fact16_tile(variant);
     if (precision == FEW_PRECISION_MIXED16 && (stage & 1) && !(stage & 2)) {
         // the spline scratch shares the region of the coefficient tiles: what

@@ -20,7 +20,7 @@ struct WaveDesc {
     int mode_off;         // first mode: sum of K before
     int cell_off;         // first cell_start entry: b * (Nr*Nc + 1)
     int ent_off;          // first gather entry
-    int pad_;
+    int dcell_off;        // FP64 direct sum: this waveform's cell count, then its cell starts
     double dt;
     long t_off;           // knot times (L)
     long teuk_off;        // knot amplitudes, complex (L, K) -> doubles
@@ -55,6 +55,8 @@ struct BatchDev {
     const int *cell_start;    // (B * (Nr*Nc + 1),)
     const int *entries;
     const int *m, *k, *n;     // concatenated mode indices (sum K)
+    const int *dcell_start;   // per waveform: number of cells, then their starts (cells.hpp)
+    const int *dcell_member;  // (sum K,) modes of the cells, at mode_off
     FactPlanDev uni;          // union grid (row tables); K, cell_start, entries unused
 };
 

@@ -237,6 +237,15 @@ int prep_stage(bool prepares, bool sums, const PrepKey &k, const char *what)
     return sums ? prep_check(k, what) : FEW_OK;
 }
 
+// Cells of a mode set, in the workspace behind `off`.  Small sets, and a
+// workspace without room for the index, run ungrouped (one cell per mode).
+static int group_modes(const int *m, const int *k, const int *n, int K, char *ws, size_t ws_bytes,
+                       size_t off, CellIndex &cells, hipStream_t stream)
+{
+    if (K < CELL_MIN_MODES || ws_bytes < off + cell_index_bytes(K)) return FEW_OK;
+    return launch_cell_index(m, k, n, K, nullptr, nullptr, 0, ws + off, cells, stream);
+}
+
 // Plans (device) and runs one waveform's mode sum on `stream`; h_t and pt
 // are device pointers.  stage: 1 = plan (+ coefficient tiles), 2 = sum,
 // 4 (with 2) = overwrite: the output is written rather than added to, and
@@ -390,7 +399,7 @@ static int run_waveform(double2 *wave, const double *interp, const double *pt, c
         set_error("get_waveform: precision %d is not supported", precision);
         return FEW_ERR_UNSUPPORTED;
     }
-    const int tile = direct_tile(precision);
+    const int tile = direct_tile(out_len);
     const PrepKey key{ws, plan, precision, tile, L, out_len};
     if (int rc = prep_stage(stage & 1, stage & 2, key, "get_waveform")) return rc;
     if (stage & 1) {
@@ -399,10 +408,6 @@ static int run_waveform(double2 *wave, const double *interp, const double *pt, c
         if (rc) return rc;
     }
     if (!(stage & 2)) return FEW_OK;
-    if (stage & 4) {
-        int rc = launch_zero_complex(wave, out_len, stream);
-        if (rc) return rc;
-    }
     DirectArgs a;
     a.wave = wave;
     a.interp = interp;
@@ -417,12 +422,16 @@ static int run_waveform(double2 *wave, const double *interp, const double *pt, c
     a.L = L;
     a.K = K;
     a.dt = dt;
+    a.out_len = out_len;
+    a.overwrite = (stage & 4) ? 1 : 0;
     const long max_blocks = ((long)out_len + tile - 1) / tile + (L - 1);
     if (max_blocks > 0x7fffffffL) {
         set_error("get_waveform: output too long (%d samples)", out_len);
         return FEW_ERR_LIMIT;
     }
-    return launch_direct_fp64(a, (int)max_blocks, stream);
+    // part of the sum, not of the preparation: the mode arrays are this call's
+    if (int rc = group_modes(m, k, n, K, ws, ws_bytes, pl.total, a.cells, stream)) return rc;
+    return launch_direct_fp64(a, tile, (int)max_blocks, stream);
 }
 
 // ------------------------------------------------------------------ adjoint
@@ -595,9 +604,8 @@ int few_prepare_modes_async(const double *teuk, const double *phase_knots, const
 size_t few_waveform_workspace_bytes(int init_len, int out_len, int num_modes, int precision)
 {
     (void)out_len;
-    (void)num_modes;
-    (void)precision;
-    return plan_layout(init_len < 2 ? 2 : init_len).total;
+    const size_t plan = plan_layout(init_len < 2 ? 2 : init_len).total;
+    return precision == FEW_PRECISION_FP64 ? plan + cell_index_bytes(num_modes) : plan;
 }
 
 int few_get_waveform(void *d_waveform, double *interp_array, double *phase_interp_t,
@@ -619,8 +627,9 @@ int few_get_waveform(void *d_waveform, double *interp_array, double *phase_inter
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     std::lock_guard<std::mutex> lk(g_ws_mu);
     const PlanLayout pl = plan_layout(init_len);
+    const size_t need = pl.total + cell_index_bytes(num_teuk_modes);
     void *ws = nullptr;
-    rc = library_workspace(cur, pl.total, &ws);
+    rc = library_workspace(cur, need, &ws);
     if (rc) return rc;
     char *w = static_cast<char *>(ws);
     // h_t and phase_interp_t are host arrays in the reference interface
@@ -632,7 +641,7 @@ int few_get_waveform(void *d_waveform, double *interp_array, double *phase_inter
                       reinterpret_cast<double *>(w + pl.pt), phase_interp_coeffs, d_m, d_k, d_n,
                       init_len, out_len, num_teuk_modes, static_cast<const double2 *>(d_Ylms),
                       delta_t, reinterpret_cast<double *>(w + pl.h_t), FEW_PRECISION_FP64, w,
-                      pl.total, s);
+                      need, s);
     if (rc) return rc;
     FEW_HIP(hipStreamSynchronize(s));
     return FEW_OK;
@@ -746,6 +755,8 @@ size_t few_plan_workspace_bytes(const void *plan, int init_len, int out_len, int
                  precision == FEW_PRECISION_FACT64)) {
         const FactPlanHost &h = static_cast<const FactPlan *>(plan)->host;
         if (h.ok) b = fact_ws_bytes(h, L, precision);
+    } else if (plan && precision == FEW_PRECISION_FP64) {
+        b += cell_index_bytes(static_cast<const FactPlan *>(plan)->host.K);
     }
     return b;
 }
@@ -1370,7 +1381,10 @@ int few_get_waveform_plan_noalloc(void *d_waveform, const double *interp_array,
     int rc = check_mode_args(d_waveform, interp_array, phase_interp_coeffs, d_m, d_k, d_n, init_len,
                              out_len, num_teuk_modes, d_Ylms, delta_t);
     if (rc) return rc;
-    const size_t need = few_plan_workspace_bytes(plan, init_len, out_len, precision);
+    // the FP64 sum needs the interval plan only (its mode index is optional)
+    const size_t need = precision == FEW_PRECISION_FP64
+                            ? plan_layout(init_len).total
+                            : few_plan_workspace_bytes(plan, init_len, out_len, precision);
     if (need > FEW_NOALLOC_SCRATCH_BYTES) {
         set_error("get_waveform_plan_noalloc: needs %zu bytes of workspace, more than the %u of "
                   "the library's scratch array (use few_get_waveform_plan_async with a caller "

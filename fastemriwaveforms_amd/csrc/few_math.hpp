@@ -158,6 +158,50 @@ __host__ __device__ inline bool sincos_cw(double x, double &s, double &c)
     return true;
 }
 
+// sin and cos of x (radians) for loops that need many of them: Cody-Waite
+// reduction to half turns, x = k pi + r with |r| <= pi/2 (twice sincos_cw's
+// constants, k up to 2^25), so the result is rotated by one sign and needs no
+// swap of sin and cos.  sin r = r + r u S(u), cos r = 1 + u C(u), u = r^2, S and
+// C Chebyshev interpolants of degree 7 and 8 on [0, pi^2/4] (errors 1.4e-18 and
+// 2.7e-19), so the polynomials are no longer than sincos_poly's quarter-turn
+// Taylor series; absolute error below 2.4e-16 measured.  Returns whether x is in range
+// (the values are meaningless if not): the caller redoes the rare tile beyond
+// it with the library routine, which keeps that routine out of its loop.
+__host__ __device__ inline bool sincos_half_turns(double x, double &s, double &c)
+{
+    const double k = rint(x * 0.31830988618379067154);  // 1/pi
+    double r = fma(-k, 3.1415926218032836914, x);        // 2 P1
+    r = fma(-k, 3.1786509424591713e-08, r);              // 2 P2
+    r = fma(-k, 1.2246467991473532e-16, r);              // 2 P3
+    const double u = r * r;
+    double ps = fma_cs(u, 2.731286399249188e-15, -7.64395589068585e-13);
+    ps = fma_cs(u, ps, 1.6058976794672544e-10);
+    ps = fma_cs(u, ps, -2.5052107607707586e-08);
+    ps = fma_cs(u, ps, 2.755731921907685e-06);
+    ps = fma_cs(u, ps, -0.0001984126984125458);
+    ps = fma_cs(u, ps, 0.008333333333333316);
+    ps = fma_cs(u, ps, -0.16666666666666666);
+    double pc = fma_cs(u, -1.5169116073483468e-16, 4.777423826499122e-14);
+    pc = fma_cs(u, pc, -1.1470695590423812e-11);
+    pc = fma_cs(u, pc, 2.087675628968416e-09);
+    pc = fma_cs(u, pc, -2.7557319218396985e-07);
+    pc = fma_cs(u, pc, 2.4801587301563063e-05);
+    pc = fma_cs(u, pc, -0.001388888888888884);
+    pc = fma_cs(u, pc, 0.041666666666666664);
+    const double sn = fma(r * u, ps, r);
+    const double cs = fma(u, fma(u, pc, -0.5), 1.0);
+    // (-1)^k
+    const unsigned long long sign = (unsigned long long)(unsigned)(int)k << 63;
+#if defined(__HIP_DEVICE_COMPILE__)
+    s = __longlong_as_double(__double_as_longlong(sn) ^ sign);
+    c = __longlong_as_double(__double_as_longlong(cs) ^ sign);
+#else
+    s = sign ? -sn : sn;
+    c = sign ? -cs : cs;
+#endif
+    return fabs(k) <= 33554432.0;  // 2^25
+}
+
 // Angle in turns reduced to [-1/2, 1/2]: a - rint(a).
 __host__ __device__ inline double reduce_turns(double a) { return a - rint(a); }
 

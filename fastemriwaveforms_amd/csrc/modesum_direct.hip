@@ -7,18 +7,17 @@
 //     interval, so one launch covers every interval (the reference launches
 //     once per interval with a device sync after each, interpolate.cu:750-771).
 //   * direct_fp64_kernel -- the plain FP64 mode sum of make_waveform
-//     (interpolate.cu:444-689): per output sample, for every mode, a cubic
-//     amplitude, the phase m*Phi_phi + k*Phi_theta + n*Phi_r, one FP64 sincos
-//     and three complex products.  Modes are staged through LDS in chunks,
-//     each lane owns SPT samples, the waveform is accumulated into without
-//     atomics (every sample belongs to exactly one lane of one block).
+//     (interpolate.cu:444-689), one term per cell (modes sharing (m, k, n),
+//     cells.hpp): per output sample and cell the phase m*Phi_phi + k*Phi_theta
+//     + n*Phi_r, one FP64 sincos and four real cubics.  The waveform is
+//     accumulated into without atomics (every sample belongs to exactly one
+//     lane of one block).
 //
 // Precision policy: the phase pipeline (dense-output evaluation, s, the
 // m/k/n combination) is evaluated with contraction off in exactly the
 // oracle's operation order, so the argument of sincos is bit-identical to
-// the CPU restatement.  Amplitude and complex products may use FMA.
-// Mode partial sums are flushed into the output every 5000 modes, matching
-// the reference CPU chunking (interpolate.cu:22, 554-600, 682-685).
+// the CPU restatement.  Amplitudes, their sums over the modes of a cell and
+// the products may use FMA.
 
 #include "batch.hpp"
 #include "few_common.hpp"
@@ -92,113 +91,163 @@ __device__ __forceinline__ int find_segment(const int *prefix, int nseg, int b)
     return lo;
 }
 
-#define MCH 256          // modes staged per LDS chunk
-#define CPU_CHUNK 5000   // interpolate.cu:22
+#define CELL_CH 64       // cells staged per LDS chunk
 
-// One 256*SPT-sample tile (tile q of interval j) of the FP64 direct sum.
-template <int SPT>
-__device__ void direct_fp64_tile(const DirectArgs &a, int j, int q)
+// One tile (64 SPT samples, tile q of interval j) of the FP64 direct sum: the
+// four waves of the workgroup hold the same samples and take every fourth cell
+// each, in a fixed order, and their partial sums are added at the end, so the
+// result of a sample depends on neither the tile size nor the output length.
+// Cells are staged CELL_CH at a time: a thread forms one power of one cell's
+// combined cubics (cell_coef_add over its modes), wave w power w, so the loads
+// of consecutive cells are consecutive modes.
+//
+// What bounds it: FP64 VALU issue, 52 instructions per (sample, cell), 30 of them
+// the sincos.  One year at 10 s, 3843 modes (671 cells): 3.6 ms, 90 % of the
+// VALU issue rate these take (33.7 ms with one term per mode, a sincos with a
+// quarter-turn swap and the library's large-argument path inside the loop).
+// Four samples per lane amortise the staging and the LDS reads (one: 6.0 ms,
+// two: 4.4 ms, the same arithmetic).
+struct DirectLds {
+    double4 c[4][CELL_CH];  // [power][cell] (P, Q, R, S)
+    double mkn[3][CELL_CH];
+};
+
+// The cell loop of a tile: this wave's partial sums (re, im) of its samples.
+// Returns whether every phase was within sincos_half_turns' range (always, if BIG).
+template <int SPT, bool BIG>
+__device__ __forceinline__ bool direct_cells(const DirectArgs &a, int j, DirectLds &sh,
+                                             const double (&x)[SPT], const double (&Pp)[SPT],
+                                             const double (&Pt)[SPT], const double (&Pr)[SPT],
+                                             double (&re)[SPT], double (&im)[SPT])
 {
-    __shared__ double sh[15][MCH];
     const int tid = threadIdx.x;
-    const Segment sg = a.segs[j];
-
-    const long np = (long)a.nseg * 3;
-    double rp[8], rt[8], rr[8];
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-        rp[c] = a.pcoef[c * np + (long)j * 3 + 0];
-        rt[c] = a.pcoef[c * np + (long)j * 3 + 1];
-        rr[c] = a.pcoef[c * np + (long)j * 3 + 2];
-    }
-
-    int idx[SPT];
-    bool ok[SPT];
-    double x[SPT], x2[SPT], x3[SPT], Pp[SPT], Pt[SPT], Pr[SPT];
-    double w_re[SPT], w_im[SPT], tr_re[SPT], tr_im[SPT];
-#pragma unroll
-    for (int u = 0; u < SPT; u++) {
-        idx[u] = sg.start + q * (256 * SPT) + u * 256 + tid;
-        ok[u] = idx[u] < sg.end;
-        SampleState st;
-        sample_state(a.dt, idx[u], sg.h_t, sg.pt, sg.pw, rp, rt, rr, st);
-        x[u] = st.x; x2[u] = st.x2; x3[u] = st.x3;
-        Pp[u] = st.Pp; Pt[u] = st.Pt; Pr[u] = st.Pr;
-        w_re[u] = 0.0; w_im[u] = 0.0;
-        if (ok[u]) {
-            const double2 w = a.wave[idx[u]];
-            w_re[u] = w.x;
-            w_im[u] = w.y;
-        }
-        tr_re[u] = 0.0;
-        tr_im[u] = 0.0;
-    }
-
+    const int part = __builtin_amdgcn_readfirstlane(tid >> 6);  // power staged, cells summed
+    const int own = tid & 63;                                   // cell staged
     const int K = a.K;
     const long nb = (long)a.L * 2 * K;
-    for (int c0 = 0; c0 < K; c0 += MCH) {
-        const int cnt = (K - c0) < MCH ? (K - c0) : MCH;
+    const double *ip = a.interp + (long)part * nb + (long)j * 2 * K;
+    const int ncell = a.cells.start ? *a.cells.count : K;
+    bool ok = true;
+#pragma unroll
+    for (int u = 0; u < SPT; u++) re[u] = im[u] = 0.0;
+    for (int c0 = 0; c0 < ncell; c0 += CELL_CH) {
+        const int cnt = min(CELL_CH, ncell - c0);
         __syncthreads();
-        if (tid < cnt) {
-            const int mode = c0 + tid;
-            const long br = (long)j * 2 * K + mode;
-            const long bi = br + K;
-            sh[0][tid] = a.interp[br];
-            sh[1][tid] = a.interp[nb + br];
-            sh[2][tid] = a.interp[2 * nb + br];
-            sh[3][tid] = a.interp[3 * nb + br];
-            sh[4][tid] = a.interp[bi];
-            sh[5][tid] = a.interp[nb + bi];
-            sh[6][tid] = a.interp[2 * nb + bi];
-            sh[7][tid] = a.interp[3 * nb + bi];
-            const double2 yp = a.ylm[mode];
-            const double2 ym = a.ylm[K + mode];
-            sh[8][tid] = yp.x;
-            sh[9][tid] = yp.y;
-            sh[10][tid] = ym.x;
-            sh[11][tid] = ym.y;
-            sh[12][tid] = (double)a.m[mode];
-            sh[13][tid] = (double)a.k[mode];
-            sh[14][tid] = (double)a.n[mode];
+        if (own < cnt) {
+            int s0 = c0 + own, s1 = s0 + 1;
+            if (a.cells.start) {
+                s0 = a.cells.start[c0 + own];
+                s1 = a.cells.start[c0 + own + 1];
+            }
+            const int lead = a.cells.start ? a.cells.member[s0] : s0;
+            const int m = a.m[lead];
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
+            for (int s = s0; s < s1; s++) {
+                const int mode = a.cells.start ? a.cells.member[s] : s;
+                const double2 yp = a.ylm[mode], ym = a.ylm[K + mode];
+                cell_coef_add(ip[mode], ip[K + mode], yp.x, yp.y, ym.x, ym.y, m != 0, v);
+            }
+            sh.c[part][own] = make_double4(v[0], v[1], v[2], v[3]);
+            if (part == 0)
+                sh.mkn[0][own] = (double)m;
+            else if (part == 1)
+                sh.mkn[1][own] = (double)a.k[lead];
+            else if (part == 2)
+                sh.mkn[2][own] = (double)a.n[lead];
         }
         __syncthreads();
-        for (int jj = 0; jj < cnt; jj++) {
-            const int mode = c0 + jj;
-            if (mode > 0 && (mode % CPU_CHUNK) == 0) {
+        for (int jj = part; jj < cnt; jj += 4) {
+            double c[4][4];
 #pragma unroll
-                for (int u = 0; u < SPT; u++) {
-                    w_re[u] = w_re[u] + tr_re[u];
-                    w_im[u] = w_im[u] + tr_im[u];
-                    tr_re[u] = 0.0;
-                    tr_im[u] = 0.0;
-                }
+            for (int p = 0; p < 4; p++) {
+                const double4 t = sh.c[p][jj];
+                c[p][0] = t.x;
+                c[p][1] = t.y;
+                c[p][2] = t.z;
+                c[p][3] = t.w;
             }
-            ModeCoef mc;
-            mc.ry = sh[0][jj]; mc.rc1 = sh[1][jj]; mc.rc2 = sh[2][jj]; mc.rc3 = sh[3][jj];
-            mc.iy = sh[4][jj]; mc.ic1 = sh[5][jj]; mc.ic2 = sh[6][jj]; mc.ic3 = sh[7][jj];
-            mc.yp_re = sh[8][jj]; mc.yp_im = sh[9][jj];
-            mc.ym_re = sh[10][jj]; mc.ym_im = sh[11][jj];
-            mc.m = sh[12][jj]; mc.k = sh[13][jj]; mc.n = sh[14][jj];
+            const double m = sh.mkn[0][jj], k = sh.mkn[1][jj], n = sh.mkn[2][jj];
 #pragma unroll
-            for (int u = 0; u < SPT; u++)
-                mode_term_fp64(mc, x[u], x2[u], x3[u], Pp[u], Pt[u], Pr[u], tr_re[u], tr_im[u]);
+            for (int u = 0; u < SPT; u++) {
+                const bool in = cell_term_fp64<BIG>(c, m, k, n, x[u], Pp[u], Pt[u], Pr[u], re[u],
+                                                    im[u]);
+                ok = ok && in;
+            }
         }
     }
+    return ok;
+}
+
+template <int SPT>
+__device__ __forceinline__ void direct_fp64_tile(const DirectArgs &a, int j, int q)
+{
+    __shared__ DirectLds sh;
+    __shared__ double2 s_sum[3][64 * SPT];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int part = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Segment sg = a.segs[j];
+    const int base = sg.start + q * (64 * SPT) + lane;
+    double x[SPT], Pp[SPT], Pt[SPT], Pr[SPT], re[SPT], im[SPT];
+    {
+        const long np = (long)a.nseg * 3;
+        double rp[8], rt[8], rr[8];
 #pragma unroll
-    for (int u = 0; u < SPT; u++) {
-        if (ok[u]) {
-            double2 w;
-            w.x = w_re[u] + tr_re[u];
-            w.y = w_im[u] + tr_im[u];
-            a.wave[idx[u]] = w;
+        for (int c = 0; c < 8; c++) {
+            rp[c] = a.pcoef[c * np + (long)j * 3 + 0];
+            rt[c] = a.pcoef[c * np + (long)j * 3 + 1];
+            rr[c] = a.pcoef[c * np + (long)j * 3 + 2];
+        }
+#pragma unroll
+        for (int u = 0; u < SPT; u++) {
+            SampleState st;
+            // samples past the interval repeat its last one (their sums are dropped)
+            sample_state(a.dt, min(base + u * 64, sg.end - 1), sg.h_t, sg.pt, sg.pw, rp, rt, rr, st);
+            x[u] = st.x;
+            Pp[u] = st.Pp;
+            Pt[u] = st.Pt;
+            Pr[u] = st.Pr;
+        }
+    }
+    const bool ok = direct_cells<SPT, false>(a, j, sh, x, Pp, Pt, Pr, re, im);
+    // phases beyond 1e8 rad (or NaN): the tile again with the library's sincos
+    if (__syncthreads_or(!ok)) direct_cells<SPT, true>(a, j, sh, x, Pp, Pt, Pr, re, im);
+    if (part > 0) {
+#pragma unroll
+        for (int u = 0; u < SPT; u++) s_sum[part - 1][u * 64 + lane] = make_double2(re[u], im[u]);
+    }
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll
+        for (int u = 0; u < SPT; u++) {
+            const int idx = base + u * 64;
+            if (idx >= sg.end) continue;
+            const double2 s1 = s_sum[0][u * 64 + lane], s2 = s_sum[1][u * 64 + lane];
+            const double2 s3 = s_sum[2][u * 64 + lane];
+            double2 w = make_double2((re[u] + s1.x) + (s2.x + s3.x), (im[u] + s1.y) + (s2.y + s3.y));
+            if (!a.overwrite) {
+                const double2 o = a.wave[idx];
+                w.x += o.x;
+                w.y += o.y;
+            }
+            a.wave[idx] = w;
         }
     }
 }
 
+// Overwriting sum: samples past the last interval's are zero.
+__device__ __forceinline__ void direct_zero_tail(const DirectArgs &a, long block, long blocks)
+{
+    const long end = a.nseg > 0 ? a.segs[a.nseg - 1].end : 0;
+    for (long i = end + block * blockDim.x + threadIdx.x; i < a.out_len; i += blocks * blockDim.x)
+        a.wave[i] = make_double2(0.0, 0.0);
+}
+
+// Four waves per SIMD (at most 128 registers)
 template <int SPT>
-__global__ __launch_bounds__(256) void direct_fp64_kernel(DirectArgs a)
+__global__ __launch_bounds__(256, 4) void direct_fp64_kernel(DirectArgs a)
 {
     const int b = blockIdx.x;
+    if (a.overwrite) direct_zero_tail(a, b, gridDim.x);
     const int total = a.prefix[a.nseg];
     if (b >= total) return;
     const int j = find_segment(a.prefix, a.nseg, b);
@@ -260,7 +309,7 @@ int launch_batch_plan(const BatchDev &B, const BatchRunDev &r, const BatchPtrs &
 
 // FP64 control run over the batch: block -> (waveform, interval, tile).
 template <int SPT>
-__global__ __launch_bounds__(256) void batch_direct_fp64_kernel(BatchDev B, BatchRunDev r,
+__global__ __launch_bounds__(256, 4) void batch_direct_fp64_kernel(BatchDev B, BatchRunDev r,
                                                                 BatchPtrs p)
 {
     const int g = blockIdx.x;
@@ -284,6 +333,13 @@ __global__ __launch_bounds__(256) void batch_direct_fp64_kernel(BatchDev B, Batc
     a.L = d.L;
     a.K = d.K;
     a.dt = d.dt;
+    if (d.K >= CELL_MIN_MODES) {
+        a.cells.count = B.dcell_start + d.dcell_off;
+        a.cells.start = a.cells.count + 1;
+        a.cells.member = B.dcell_member + d.mode_off;
+    }
+    a.out_len = d.N;
+    a.overwrite = 0;
     direct_fp64_tile<SPT>(a, j, lt - pref[j]);
 }
 
@@ -291,8 +347,8 @@ int launch_batch_direct_fp64(const BatchDev &B, const BatchRunDev &r, const Batc
                              int max_blocks, hipStream_t stream)
 {
     if (max_blocks <= 0) return FEW_OK;
-    hipLaunchKernelGGL(batch_direct_fp64_kernel<DIRECT_SPT>, dim3(max_blocks), dim3(256), 0, stream,
-                       B, r, p);
+    hipLaunchKernelGGL(batch_direct_fp64_kernel<DIRECT_SPT>, dim3(max_blocks),
+                       dim3(256), 0, stream, B, r, p);
     FEW_HIP(hipGetLastError());
     return FEW_OK;
 }
@@ -308,12 +364,22 @@ int launch_plan(const PlanArgs &p, hipStream_t stream)
     return FEW_OK;
 }
 
-int direct_tile(int /*precision*/) { return 256 * DIRECT_SPT; }
+// Below 2^17 samples the four-sample tiles are too few to fill the chip: 63,116
+// samples of the full set take 128 us with one sample per lane and 183 us with
+// four, 315,582 samples of 500 modes 193 us with four and 217 us with one.
+int direct_tile(long out_len)
+{
+    return out_len < (1L << 17) ? 64 : DIRECT_TILE;
+}
 
-int launch_direct_fp64(const DirectArgs &a, int max_blocks, hipStream_t stream)
+int launch_direct_fp64(const DirectArgs &a, int tile, int max_blocks, hipStream_t stream)
 {
     if (max_blocks <= 0) return FEW_OK;
-    hipLaunchKernelGGL(direct_fp64_kernel<DIRECT_SPT>, dim3(max_blocks), dim3(256), 0, stream, a);
+    const dim3 grid(max_blocks);
+    if (tile == DIRECT_TILE)
+        hipLaunchKernelGGL(direct_fp64_kernel<DIRECT_SPT>, grid, dim3(256), 0, stream, a);
+    else
+        hipLaunchKernelGGL(direct_fp64_kernel<1>, grid, dim3(256), 0, stream, a);
     FEW_HIP(hipGetLastError());
     return FEW_OK;
 }

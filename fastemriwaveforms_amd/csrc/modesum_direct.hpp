@@ -4,12 +4,9 @@
 
 #include <math.h>
 
+#include "cells.hpp"
 #include "few_common.hpp"
 #include "few_math.hpp"
-
-#ifndef DIRECT_SPT
-#define DIRECT_SPT 2  // output samples per lane in the FP64 direct kernel
-#endif
 
 namespace few {
 
@@ -36,6 +33,9 @@ struct DirectArgs {
     int L;
     int K;
     double dt;
+    CellIndex cells;          // modes sharing (m, k, n); ungrouped: one cell per mode
+    int out_len;
+    int overwrite;            // write the samples (0 where no interval has any) instead of adding
 };
 
 // Output sample index -> start of its interval, find_start_inds rule
@@ -154,8 +154,53 @@ __host__ __device__ inline void mode_term_fp64(const ModeCoef &c, double x, doub
     tr_im = tr_im + tm_im + tp_im;
 }
 
+// The same contribution for all modes of one cell (one phase): with the cubics
+// C+ = sum Y+ A and C- = sum Y- conj(A) (m != 0) of its members,
+//   C+ exp(-i phase) + C- exp(+i phase)
+//     = (P cos + Q sin) + i (R cos + S sin),
+//   P = Re C+ + Re C-, Q = Im C+ - Im C-, R = Im C+ + Im C-, S = Re C- - Re C+.
+// cell_coef_add adds a member's power p to (P, Q, R, S) of that power.
+__host__ __device__ inline void cell_coef_add(double a_re, double a_im, double yp_re, double yp_im,
+                                              double ym_re, double ym_im, bool minus, double (&v)[4])
+{
+    const double p_re = a_re * yp_re - a_im * yp_im, p_im = a_re * yp_im + a_im * yp_re;
+    const double m_re = minus ? a_re * ym_re + a_im * ym_im : 0.0;
+    const double m_im = minus ? a_re * ym_im - a_im * ym_re : 0.0;
+    v[0] += p_re + m_re;
+    v[1] += p_im - m_im;
+    v[2] += p_im + m_im;
+    v[3] += m_re - p_re;
+}
+
+// Sample term of one cell; c[p] holds (P, Q, R, S) of power p.  BIG: any phase
+// (the library's sincos beyond sincos_cw's range); otherwise sincos_half_turns, and returns whether
+// the phase was within that range (the term is meaningless if not).
+template <bool BIG>
+__host__ __device__ inline bool cell_term_fp64(const double (&c)[4][4], double m, double k, double n,
+                                               double x, double Pp, double Pt, double Pr,
+                                               double &tr_re, double &tr_im)
+{
+    const double phase = mode_phase(m, Pp, k, Pt, n, Pr);
+    double sn, cs;
+    bool ok = true;
+    if (BIG) {
+        if (!sincos_cw(phase, sn, cs)) sincos(phase, &sn, &cs);
+    } else {
+        ok = sincos_half_turns(phase, sn, cs);
+    }
+    double v[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = fma(fma(fma(c[3][e], x, c[2][e]), x, c[1][e]), x, c[0][e]);
+    tr_re = fma(v[0], cs, fma(v[1], sn, tr_re));
+    tr_im = fma(v[2], cs, fma(v[3], sn, tr_im));
+    return ok;
+}
+
 int launch_plan(const PlanArgs &p, hipStream_t stream);
-int direct_tile(int precision);
-int launch_direct_fp64(const DirectArgs &a, int max_blocks, hipStream_t stream);
+constexpr int DIRECT_SPT = 4;                  // output samples per lane of a tile
+constexpr int DIRECT_TILE = 64 * DIRECT_SPT;
+// Samples per tile of the FP64 direct sum for an output of out_len samples.
+int direct_tile(long out_len);
+int launch_direct_fp64(const DirectArgs &a, int tile, int max_blocks, hipStream_t stream);
 
 }  // namespace few

@@ -380,4 +380,26 @@ void twin_sincos_turns(const double *f, double *s, double *c, long n)
     for (long i = 0; i < n; i++) sincos_turns(reduce_turns(f[i]), s[i], c[i]);
 }
 
+void twin_sincos_half_turns(const double *x, double *s, double *c, int *ok, long n)
+{
+    for (long i = 0; i < n; i++) ok[i] = sincos_half_turns(x[i], s[i], c[i]) ? 1 : 0;
+}
+
+// One sample of one cell: the members' combined cubics, then the cell's term
+// (big: its any-phase form).
+void twin_cell_term(int members, const double *coef, const double *ylm, double m, double k, double n,
+                    double x, double Pp, double Pt, double Pr, int big, double *out)
+{
+    double c[4][4] = {};
+    for (int q = 0; q < members; q++)
+        for (int p = 0; p < 4; p++)
+            cell_coef_add(coef[8 * q + p], coef[8 * q + 4 + p], ylm[4 * q], ylm[4 * q + 1],
+                          ylm[4 * q + 2], ylm[4 * q + 3], m != 0.0, c[p]);
+    out[0] = out[1] = 0.0;
+    if (big)
+        cell_term_fp64<true>(c, m, k, n, x, Pp, Pt, Pr, out[0], out[1]);
+    else
+        cell_term_fp64<false>(c, m, k, n, x, Pp, Pt, Pr, out[0], out[1]);
+}
+
 }  // extern "C"
