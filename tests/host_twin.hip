@@ -14,6 +14,7 @@
 
 #include "spline.hip"
 #include "adjoint.hip"
+#include "cells.hip"
 #include "fd.hip"
 #include "amp2d.hip"
 #include "aak.hip"
@@ -400,6 +401,93 @@ void twin_cell_term(int members, const double *coef, const double *ylm, double m
         cell_term_fp64<true>(c, m, k, n, x, Pp, Pt, Pr, out[0], out[1]);
     else
         cell_term_fp64<false>(c, m, k, n, x, Pp, Pt, Pr, out[0], out[1]);
+}
+
+// twin_fd_waveform with the kernels' form of a bin (fd_bin_fast): summed output
+// only, the modes one by one.
+int twin_fd_waveform_fast(double *wave, const double *interp, const double *phase_t,
+                          const double *pcoef, const int *m, const int *k, const int *n, int K,
+                          const double *t_knots, int L, int Nf, const double *freqs,
+                          const int *seg_start, const int *seg_end, int nseg, const double *ylm,
+                          int zero_index, int include_minus_m)
+{
+    FdArgs a{};
+    a.interp = interp;
+    a.phase_t = phase_t;
+    a.pcoef = pcoef;
+    a.m = m;
+    a.k = k;
+    a.n = n;
+    a.t_knots = t_knots;
+    a.seg_start = seg_start;
+    a.seg_end = seg_end;
+    a.K = K;
+    a.L = L;
+    a.nseg = nseg;
+    a.data_length = Nf;
+    const double2 *y = reinterpret_cast<const double2 *>(ylm);
+    const FdSpaConst kc = fd_spa_const();
+    const FdRootConst kr = fd_root_const();
+    const long nb = (2L * K + 3) * L;
+    for (int q = 0; q < K; q++)
+        for (int j = 0; j < nseg; j++) {
+            int lo, hi;
+            fd_item_range(a, (long)q * nseg + j, lo, hi);
+            if (hi < lo) continue;
+            FdSeg it;
+            fd_load_seg(a, q, j, it);
+            fcx cp[4] = {}, cm[4] = {};
+            for (int p = 0; p < 4; p++)
+                fd_cell_add(interp[p * nb + (long)q * L + j], interp[p * nb + (long)(K + q) * L + j],
+                            y[q], y[K + q], cp[p], cm[p]);
+            for (int i = lo; i <= hi; i++)
+                fd_bin_fast(it, freqs[i], kr, kc, [&](double x, fcx B) {
+                    fcx P = cp[3], M = cm[3];
+                    for (int p = 2; p >= 0; p--) {
+                        P = fcx_add(fcx_scale(P, x), cp[p]);
+                        M = fcx_add(fcx_scale(M, x), cm[p]);
+                    }
+                    wave[2L * i] += P.re * B.re - P.im * B.im;
+                    wave[2L * i + 1] += P.re * B.im + P.im * B.re;
+                    const int mi = fd_minus_index(zero_index, i);
+                    if (include_minus_m && m[q] != 0 && mi >= 0 && mi < Nf) {
+                        wave[2L * mi] += M.re * B.re + M.im * B.im;
+                        wave[2L * mi + 1] += M.im * B.re - M.re * B.im;
+                    }
+                });
+        }
+    return 0;
+}
+
+// fd_amp, and fd_bin's form of the same factor
+void twin_fd_amp(const double *fdot, const double *fddot, long n, double *fast, double *ref)
+{
+    const FdSpaConst kc = fd_spa_const();
+    for (long i = 0; i < n; i++) {
+        const fcx f = fd_amp(fdot[i], fddot[i], kc), r = fd_amp_any(fdot[i], fddot[i], kc);
+        fast[2 * i] = f.re;
+        fast[2 * i + 1] = f.im;
+        ref[2 * i] = r.re;
+        ref[2 * i + 1] = r.im;
+    }
+}
+
+// fd_cube_c / fd_root_of in the place of fd_cube_roots
+void twin_fd_roots(const double *abcd, long n, double *out)
+{
+    for (long i = 0; i < n; i++) {
+        const double a = abcd[4 * i], b = abcd[4 * i + 1], c = abcd[4 * i + 2];
+        FdSeg it{};
+        it.b = b;
+        it.D0 = b * b - 3 * a * c;
+        it.D03 = 4 * (it.D0 * it.D0 * it.D0);
+        it.D1c = 2 * (b * b * b) - 9 * a * b * c;
+        it.a27 = 27 * (a * a);
+        it.a = -(1. / (3 * a));
+        fcx C[3];
+        fd_cube_c(it, abcd[4 * i + 3], fd_root_const(), C);
+        for (int k = 0; k < 3; k++) out[3 * i + k] = fd_root_of(it, C[k]);
+    }
 }
 
 }  // extern "C"
