@@ -29,6 +29,15 @@ def frequency_grid(num_pts: int, num_pts_pad: int, dt: float) -> np.ndarray:
     return np.hstack((np.arange(-(Len // 2), 0), np.arange(0, (Len - 1) // 2 + 1))) / (Len * dt)
 
 
+def frequency_grid_device(num_pts: int, num_pts_pad: int, dt: float) -> torch.Tensor:
+    """:func:`frequency_grid` formed on the GPU, the same values: whole numbers
+    over Len * dt, a correctly rounded quotient on both sides (the divisor is a
+    tensor: a scalar one would be multiplied by its reciprocal)."""
+    Len = num_pts + num_pts_pad
+    k = torch.arange(-(Len // 2), (Len - 1) // 2 + 1, dtype=torch.float64, device=_device())
+    return k / torch.full((1,), Len * dt, dtype=torch.float64, device=k.device)
+
+
 def segment_frequency_inds(t, f_phi, f_theta, f_r, m, k, n, frequency: torch.Tensor,
                            f_arr_given: bool = False):
     """fdinterp.py:241-465: first/last frequency index of every (mode, segment).
@@ -163,8 +172,7 @@ class FDInterpolatedModeSum(SummationBase):
             if len(self.frequency) == 0:
                 raise ValueError("Input f_arr kwarg has zero length.")
         else:
-            self.frequency = torch.from_numpy(
-                frequency_grid(self.num_pts, self.num_pts_pad, dt)).to(_device())
+            self.frequency = frequency_grid_device(self.num_pts, self.num_pts_pad, dt)
         start_inds, end_inds, zero_index = segment_frequency_inds(
             t, f_phi, f_theta, f_r, m_arr, k_arr, n_arr, self.frequency,
             f_arr_given=f_arr is not None)

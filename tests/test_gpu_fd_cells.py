@@ -71,3 +71,11 @@ def test_many_segments(gpu, L):
     freq = _grid(inp)
     ref, (start, end, zero) = oracle_fd(inp, freq)
     assert _rel_l2(_run_capi(inp, freq, start, end, zero), ref) < FD_TOL
+
+
+@pytest.mark.parametrize("n,pad,dt", [(1, 0, 3.0), (2, 1, 7.3), (315581, 0, 10.0), (315582, 1, 15.0)])
+def test_frequency_grid_device(gpu, n, pad, dt):
+    """The grid formed on the GPU holds numpy's values."""
+    from fastemriwaveforms_amd import fdinterp
+    np.testing.assert_array_equal(fdinterp.frequency_grid_device(n, pad, dt).cpu().numpy(),
+                                  fdinterp.frequency_grid(n, pad, dt))
