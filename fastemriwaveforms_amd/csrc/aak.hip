@@ -9,13 +9,12 @@
 // The Bessel functions are the Numerical Recipes routines the reference's CPU
 // branch uses (rational / asymptotic J0, J1; Miller's backward recurrence for
 // J_n below its order), restated here so the device result follows the CPU
-// reference rather than a library jn.  Everything else is the reference's
-// arithmetic in its order with contraction off, on the device's FP64 libm;
-// the cos and sin of one argument are taken with one sincos call (as an
-// optimising compiler merges them), so the result does not depend on
-// whether a compiler merges the pair.
+// reference rather than a library jn.  aak_sample is the reference's arithmetic
+// in its order with contraction off, the cos and sin of one argument taken with
+// one sincos call (as an optimising compiler merges them); the kernel runs
+// aak_sample_fast, the same quantities with fewer operations.
 //
-// Work layout: a one-thread planning kernel turns the knot times into sample
+// Work layout: a one-wave planning kernel turns the knot times into sample
 // ranges with the reference's rule (gpuAAK.cu:458-483); the sum kernel runs
 // one lane per output sample over all segments in one launch (the reference
 // launches one kernel per segment on its own stream).
@@ -23,6 +22,7 @@
 
 #include "aak.hpp"
 #include "few_common.hpp"
+#include "few_math.hpp"
 
 #pragma clang fp contract(off)
 
@@ -255,18 +255,142 @@ __host__ __device__ inline void nr_jn5(int nu0, double x, double (&out)[5])
     }
 }
 
+// The rare branches of aak_bessel5, out of line: inlined, their registers and
+// library calls would set the sum kernel's.
+__host__ __device__ __attribute__((noinline)) double nr_jn_any(int n, double x) { return nr_jn(n, x); }
+struct Bessel5 {
+    double v[5];
+};
+__host__ __device__ __attribute__((noinline)) Bessel5 nr_jn5_any(int nu0, double x)
+{
+    Bessel5 r;
+    nr_jn5(nu0, x, r.v);
+    return r;
+}
+
+// nr_jn5's values from two recurrences instead of five, to rounding.
+//
+// The Miller sequence started at m is the solution of p_{k-1} = (2k/x) p_k -
+// p_{k+1} that vanishes at m + 1, and all of them are combinations of two: with
+// u started at the highest start A and w at the lowest B (continued upward to
+// the others), p = u w_{m+1} - w u_{m+1} is the one started at m, so
+//     J_n = (u_n w_{m+1} - w_n u_{m+1}) / (U w_{m+1} - W u_{m+1})
+// with U, W the normalising sums over the orders nr_jn_miller sums for that
+// start (even, up to m - 2).  w_{m+1} is negative and everything else positive:
+// no cancellation, and each value keeps the truncation of its own start (3e-7
+// for orders 2 and 3), which the reference's routines have.
+//
+// Seeds of 2^-400 and a bound on the growth (the product of 2k/x) keep every
+// product in range without the rescaling; beyond it (x below ~1e-4 n, orders in
+// the hundreds, zero or NaN) nr_jn5 runs.
+// st: nr_miller_start of the orders nu0 .. nu0 + 4, those below 2 as order 2.
+__host__ __device__ inline void aak_bessel5(int nu0, double x, const int (&st)[5], double (&out)[5])
+{
+    const int A = st[4], B = st[0];
+    // prod_{k <= A} 2k/x < 8 A^(1/2) (2 A / (e x))^A
+    if (!((float)A * log2f(0.736f * (float)A / (float)x) < 880.0f)) {
+        const Bessel5 r = nr_jn5_any(nu0, x);
+#pragma unroll
+        for (int i = 0; i < 5; i++) out[i] = r.v[i];
+        return;
+    }
+    const double two_over_x = 2.0 / x;
+    const double seed = 0x1p-400;
+    // per start m of the orders between: the base solutions at m + 1, and the part
+    // of their sums that differs from the base's own
+    double u1[3], ut[3], w1[3], wt[3];
+    {
+        double even = seed, odd = 0.0, sum = 0.0;  // w_k, w_{k+1}, even orders B .. k - 2
+        int k = B;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            for (; k < st[i + 1]; k += 2) {
+                sum += even;
+                even = fma((k + 1) * two_over_x, odd, -even);
+                odd = fma((k + 2) * two_over_x, even, -odd);
+            }
+            w1[i] = odd;
+            wt[i] = sum;
+        }
+    }
+    double u = seed, up = 0.0, ue = 0.0;  // u_k, u_{k+1}, even orders k .. A - 2
+    int k = A;
+#pragma unroll
+    for (int i = 2; i >= -1; i--) {
+        for (; k > st[i + 1]; k -= 2) {
+            up = fma(k * two_over_x, u, -up);
+            u = fma((k - 1) * two_over_x, up, -u);
+            ue += u;
+        }
+        if (i >= 0) {
+            u1[i] = up;
+            ut[i] = ue;
+        }
+    }
+    double w = seed, wp = 0.0, we = 0.0;
+    auto pair = [&]() {
+        const double k0 = k * two_over_x, k1 = (k - 1) * two_over_x;
+        up = fma(k0, u, -up);
+        wp = fma(k0, w, -wp);
+        u = fma(k1, up, -u);
+        w = fma(k1, wp, -w);
+        ue += u;
+        we += w;
+        k -= 2;
+    };
+    // down to the even order at or above nu0 + 4, three pairs over the five
+    // orders (kept from the top: six of each), the rest
+    const int top = (nu0 + 5) & ~1;
+    while (k > top) pair();
+    double uc[6], wc[6];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        uc[2 * j] = u;
+        wc[2 * j] = w;
+        if (k > 0) pair();  // up, wp: the odd order just passed
+        uc[2 * j + 1] = up;
+        wc[2 * j + 1] = wp;
+    }
+    while (k > 0) pair();
+    const bool even4 = top == nu0 + 4;  // uc[0] is order nu0 + 4, else nu0 + 5
+    out[0] = (even4 ? wc[4] : wc[5]) / fma(2.0, we, -w);
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const double un = even4 ? uc[3 - i] : uc[4 - i], wn = even4 ? wc[3 - i] : wc[4 - i];
+        const double U = fma(2.0, ue - ut[i], -u), W = fma(2.0, we + wt[i], -w);
+        out[i + 1] = fma(un, w1[i], -wn * u1[i]) / fma(U, w1[i], -W * u1[i]);
+    }
+    out[4] = (even4 ? uc[0] : uc[1]) / fma(2.0, ue, -u);
+    // orders 0 and 1 and orders below x are not Miller's (nr_jn)
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+        const int nu = nu0 + i;
+        if (nu >= 0 && (nu < 2 || x > (double)nu)) out[i] = nr_jn_any(nu, x);
+    }
+}
+
+// sin and cos of any argument: the mode sum's, the library's beyond its range.
+__host__ __device__ __attribute__((noinline)) double2 aak_sincos_any(double x)
+{
+    double2 r;
+    sincos(x, &r.x, &r.y);
+    return r;
+}
+__host__ __device__ inline void aak_sincos(double x, double *s, double *c)
+{
+    if (!sincos_half_turns(x, *s, *c)) {
+        const double2 r = aak_sincos_any(x);
+        *s = r.x;
+        *c = r.y;
+    }
+}
+
 // gpuAAK.cu:136-176: rotation coefficients source frame -> wave frame
-__host__ __device__ inline void aak_rot_coeff(double *rot, double iota, double theta_S, double phi_S,
-                                              double theta_K, double phi_K, double alpha)
+__host__ __device__ inline void aak_rot_coeff(double *rot, double sI, double cI, double sTS, double cTS,
+                                              double sPS, double cPS, double sTK, double cTK,
+                                              double sPK, double cPK, double sA, double cA)
 {
     double n[3], S[3], L[3], nxL[3], nxS[3];
-    double sTS, cTS, sPS, cPS, sTK, cTK, sPK, cPK, sI, cI, sA, cA;
-    sincos(theta_S, &sTS, &cTS);
-    sincos(phi_S, &sPS, &cPS);
-    sincos(theta_K, &sTK, &cTK);
-    sincos(phi_K, &sPK, &cPK);
-    sincos(iota, &sI, &cI);
-    sincos(alpha, &sA, &cA);
     n[0] = sTS * cPS;
     n[1] = sTS * sPS;
     n[2] = cTS;
@@ -311,24 +435,39 @@ __host__ __device__ inline double aak_dense_dot(const double *r, double s, doubl
            r[7] * (4. * s3 - 15. * s4 + 18. * s5 - 7. * s6);
 }
 
-// One output sample i of segment j (gpuAAK.cu:270-451); sc[p][c] are the
-// segment's dense coefficients.  Returns hI - i hII.
-__host__ __device__ inline double2 aak_sample(const AakArgs &a, const double (*sc)[8], double start_t,
-                                              double segwidth, long i)
+// What the sample formulas take from the source's position and spin alone.
+struct AakGeom {
+    double cosqS, sinqS, cosqK, sinqK, cosphiK, sinphiK, cosphiS, sinphiS, cosdphi, sindphi;
+};
+
+__host__ __device__ inline AakGeom aak_geom(const AakArgs &a)
 {
     double qS = a.qS, qK = a.qK;
-    const double phiS = a.phiS, phiK = a.phiK;
     const double fill_val = 1e-6;
     if (qS < fill_val) qS = fill_val;
     if (qK < fill_val) qK = fill_val;
     if (qS > M_PI - fill_val) qS = M_PI - fill_val;
     if (qK > M_PI - fill_val) qK = M_PI - fill_val;
-    double cosqS, sinqS, cosqK, sinqK, cosphiK, sinphiK, cosphiS, sinphiS, cosdphi, sindphi;
-    sincos(qS, &sinqS, &cosqS);
-    sincos(qK, &sinqK, &cosqK);
-    sincos(phiK, &sinphiK, &cosphiK);
-    sincos(phiS, &sinphiS, &cosphiS);
-    sincos(phiK - phiS, &sindphi, &cosdphi);
+    AakGeom g;
+    sincos(qS, &g.sinqS, &g.cosqS);
+    sincos(qK, &g.sinqK, &g.cosqK);
+    sincos(a.phiK, &g.sinphiK, &g.cosphiK);
+    sincos(a.phiS, &g.sinphiS, &g.cosphiS);
+    sincos(a.phiK - a.phiS, &g.sindphi, &g.cosdphi);
+    return g;
+}
+
+// One output sample i of segment j (gpuAAK.cu:270-451); sc[p][c] are the
+// segment's dense coefficients.  Returns hI - i hII, by the reference's
+// operations one for one (the host tests' form; the kernel's is below).
+__host__ __device__ inline double2 aak_sample(const AakArgs &a, const double (*sc)[8], double start_t,
+                                              double segwidth, long i)
+{
+    const AakGeom G = aak_geom(a);
+    const double phiS = a.phiS, phiK = a.phiK;
+    const double cosqS = G.cosqS, sinqS = G.sinqS, cosqK = G.cosqK, sinqK = G.sinqK;
+    const double cosphiK = G.cosphiK, sinphiK = G.sinphiK, cosphiS = G.cosphiS, sinphiS = G.sinphiS;
+    const double cosdphi = G.cosdphi, sindphi = G.sindphi;
     const double halfsqrt3 = sqrt(3.) / 2.;
     const double mu_sec = a.mu * AAK_MTSUN_SI;
     const double zeta = mu_sec / a.dist / AAK_GPCINSEC;
@@ -399,8 +538,10 @@ __host__ __device__ inline double2 aak_sample(const AakArgs &a, const double (*s
     }
     const double Amp = pow(fabs(OmegaPhi) * a.M_phys * AAK_MTSUN_SI, 2. / 3.) * zeta;
     double rot[4];
-    aak_rot_coeff(rot, lam, qS, phiS, qK, phiK, alp);
+    aak_rot_coeff(rot, sinlam, coslam, sinqS, cosqS, sinphiS, cosphiS, sinqK, cosqK, sinphiK, cosphiK,
+                  sinalp, cosalp);
     double hItemp = 0.0, hIItemp = 0.0;
+    const double sq1e = sqrt(1 - e * e);
     for (int n = 1; n <= a.nmodes; n++) {
         double nPhi;
         if (a.mich) {
@@ -413,12 +554,12 @@ __host__ __device__ inline double2 aak_sample(const AakArgs &a, const double (*s
         const double ne = n * e;
         double Jv[5];
         nr_jn5(n - 2, ne, Jv);
-        const double J0 = (n == 1) ? -1.0 * nr_j1(ne) : Jv[0];
+        const double J0 = (n == 1) ? -1.0 * Jv[2] : Jv[0];
         const double J1 = Jv[1], J2 = Jv[2], J3 = Jv[3], J4 = Jv[4];
         double sn, cn;
         sincos(nPhi, &sn, &cn);
         const double aa = -n * Amp * (J0 - 2. * e * J1 + 2. / n * J2 + 2. * e * J3 - J4) * cn;
-        const double bb = -n * Amp * sqrt(1 - e * e) * (J0 - 2. * J2 + J4) * sn;
+        const double bb = -n * Amp * sq1e * (J0 - 2. * J2 + J4) * sn;
         const double cc = 2. * Amp * J2 * cn;
         const double Aplus0 = -(1. + Ldotn2) * (aa * cos2gam - bb * sin2gam) + cc * (1 - Ldotn2);
         const double Acros0 = 2. * Ldotn * (bb * cos2gam + aa * sin2gam);
@@ -436,6 +577,130 @@ __host__ __device__ inline double2 aak_sample(const AakArgs &a, const double (*s
         hIItemp += hnII;
     }
     return make_double2(hItemp, -hIItemp);
+}
+
+// aak_sample in the kernel's form.  What the phases of 1e5-1e6 rad pass through
+// (the splines, gim + beta, n Phi + Doppler) is the same operations, as an ulp
+// there is 1e-11 and more; the rest is the same quantities with fewer of them:
+//   * the harmonics enter h through three sums over n, sum a_n, b_n and c_n,
+//     and the geometry is applied once;
+//   * lambda = acos Y, phi_L, psi and the detector angle of the source appear
+//     only through their sines and cosines, taken from the ratios their inverse
+//     functions would have been given;
+//   * Bessel values by aak_bessel5, the other sines and cosines by aak_sincos.
+__host__ __device__ inline double2 aak_sample_fast(const AakArgs &a, const AakGeom &G,
+                                                   const double (*sc)[8], double start_t,
+                                                   double segwidth, long i)
+{
+    const double cosqS = G.cosqS, sinqS = G.sinqS, cosqK = G.cosqK, sinqK = G.sinqK;
+    const double cosphiK = G.cosphiK, sinphiK = G.sinphiK, cosphiS = G.cosphiS, sinphiS = G.sinphiS;
+    const double cosdphi = G.cosdphi, sindphi = G.sindphi;
+    const double halfsqrt3 = 0.86602540378443864676;
+    const double zeta = a.mu * AAK_MTSUN_SI / a.dist / AAK_GPCINSEC;
+    const double t = a.dt * i;
+    const double s = (t - start_t) / segwidth;
+    const double s1 = (1.0 - s);
+    const double s2 = s * s, s3 = s * s2, s4 = s * s3, s5 = s * s4, s6 = s * s5;
+    const double e = aak_dense(sc[1], s, s1);
+    const double Y = aak_dense(sc[2], s, s1);
+    const double Phi_phi = aak_dense(sc[3], s, s1);
+    const double Phi_theta = aak_dense(sc[4], s, s1);
+    const double Phi_r = aak_dense(sc[5], s, s1);
+    const double OmegaPhi = aak_dense_dot(sc[3], s, s2, s3, s4, s5, s6) / segwidth;
+    const double OmegaTheta = aak_dense_dot(sc[4], s, s2, s3, s4, s5, s6) / segwidth;
+    const double OmegaR = aak_dense_dot(sc[5], s, s2, s3, s4, s5, s6) / segwidth;
+    const double gim = Phi_theta - Phi_r;
+    const double alp = Phi_phi - Phi_theta;
+    const double nu = OmegaR / (2. * M_PI);
+    const double gimdot = OmegaTheta - OmegaR;
+    const double orbphs = 2. * M_PI * t / AAK_YRSID_SI;
+    double sinorbphs = 0.0, cosorbphs = 0.0;
+    if (a.mich) aak_sincos(orbphs - a.phiS, &sinorbphs, &cosorbphs);
+    const double coslam = Y, sinlam = sqrt((1.0 - Y) * (1.0 + Y));  // NaN for |Y| > 1, as acos
+    double cosalp, sinalp;
+    aak_sincos(alp, &sinalp, &cosalp);
+    const double cosqL = cosqK * coslam + sinqK * sinlam * cosalp;
+    const double sinqL = sqrt(1. - cosqL * cosqL);
+    const double phiLup = sinqK * sinphiK * coslam - cosphiK * sinlam * sinalp - cosqK * sinphiK * sinlam * cosalp;
+    const double phiLdown = sinqK * cosphiK * coslam + sinphiK * sinlam * sinalp - cosqK * cosphiK * sinlam * cosalp;
+    const double rL = sqrt(phiLup * phiLup + phiLdown * phiLdown);
+    const double cosLS = rL == 0.0 ? cosphiS : (phiLdown * cosphiS + phiLup * sinphiS) / rL;
+    const double Ldotn = cosqL * cosqS + sinqL * sinqS * cosLS;
+    const double Ldotn2 = Ldotn * Ldotn;
+    const double Sdotn = cosqK * cosqS + sinqK * sinqS * cosdphi;
+    double beta = 0.0;
+    if (!(a.S_phys == 0.0 || sinlam < 1e-10)) {
+        const double betaup = -Sdotn + coslam * Ldotn;
+        const double betadown = sinqS * sindphi * sinlam * cosalp + (cosqK * Sdotn - cosqS) / sinqK * sinlam * sinalp;
+        beta = atan2(betaup, betadown);
+    }
+    const double gam = 2. * (gim + beta);
+    double cos2gam, sin2gam;
+    aak_sincos(gam, &sin2gam, &cos2gam);
+    double FplusI = 1.0, FcrosI = 0.0, FplusII = 0.0, FcrosII = 1.0;
+    if (a.mich) {
+        double sinorb, cosorb;
+        aak_sincos(orbphs, &sinorb, &cosorb);
+        const double cosq = .5 * cosqS - halfsqrt3 * sinqS * cosorbphs;
+        // cos and sin of twice atan2(y, x)
+        auto twice = [](double y, double x, double &c, double &sn) {
+            const double r = x * x + y * y;
+            c = r == 0.0 ? 1.0 : (x * x - y * y) / r;
+            sn = r == 0.0 ? 0.0 : 2.0 * x * y / r;
+        };
+        double ca, sa, cos2psi, sin2psi;
+        twice(halfsqrt3 * cosqS + .5 * sinqS * cosorbphs, sinqS * sinorbphs, ca, sa);
+        const double co = 1.0 - 2.0 * sinorb * sinorb, so = 2.0 * sinorb * cosorb;
+        const double cos2phi = co * ca - so * sa, sin2phi = so * ca + co * sa;
+        const double cosoK = cosorb * cosphiK + sinorb * sinphiK;
+        const double psiup = .5 * cosqK - halfsqrt3 * sinqK * cosoK - cosq * (cosqK * cosqS + sinqK * sinqS * cosdphi);
+        const double psidown = .5 * sinqK * sinqS * sindphi - halfsqrt3 * cosorb * (cosqK * sinqS * sinphiS - cosqS * sinqK * sinphiK) - halfsqrt3 * sinorb * (cosqS * sinqK * cosphiK - cosqK * sinqS * cosphiS);
+        twice(psiup, psidown, cos2psi, sin2psi);
+        const double cosq1 = .5 * (1. + cosq * cosq);
+        FplusI = halfsqrt3 * (cosq1 * cos2phi * cos2psi - cosq * sin2phi * sin2psi);
+        FcrosI = halfsqrt3 * (cosq1 * cos2phi * sin2psi + cosq * sin2phi * cos2psi);
+        FplusII = halfsqrt3 * (cosq1 * sin2phi * cos2psi + cosq * cos2phi * sin2psi);
+        FcrosII = halfsqrt3 * (cosq1 * sin2phi * sin2psi - cosq * cos2phi * cos2psi);
+    }
+    const double root = cbrt(fabs(OmegaPhi) * a.M_phys * AAK_MTSUN_SI);
+    const double Amp = root * root * zeta;
+    double rot[4];
+    aak_rot_coeff(rot, sinlam, coslam, sinqS, cosqS, sinphiS, cosphiS, sinqK, cosqK, sinphiK, cosphiK,
+                  sinalp, cosalp);
+    double sum_a = 0.0, sum_b = 0.0, sum_c = 0.0;
+    // Miller starts of the orders n - 2 .. n + 2 (order 2's for those below 2),
+    // shifted along with n; isq = floor(sqrt(40 (n + 2)))
+    int st[5], isq = 8;
+    st[0] = st[1] = st[2] = st[3] = 2 * ((2 + 8) / 2);
+    st[4] = 0;
+    for (int n = 1; n <= a.nmodes; n++) {
+        while ((isq + 1) * (isq + 1) <= 40 * (n + 2)) isq++;
+        st[4] = 2 * ((n + 2 + isq) / 2);
+        double nPhi;
+        if (a.mich) {
+            const double fn = n * nu + gimdot / M_PI;
+            const double Doppler = 2. * M_PI * fn * AAK_AUSEC * sinqS * cosorbphs;
+            nPhi = n * Phi_r + Doppler;
+        } else {
+            nPhi = n * Phi_r;
+        }
+        double J[5];
+        aak_bessel5(n - 2, n * e, st, J);
+        if (n == 1) J[0] = -J[2];
+        double sn, cn;
+        aak_sincos(nPhi, &sn, &cn);
+        sum_a = fma(fma((double)n, fma(2.0 * e, J[3] - J[1], J[0] - J[4]), 2.0 * J[2]), cn, sum_a);
+        sum_b = fma((double)n * fma(-2.0, J[2], J[0] + J[4]), sn, sum_b);
+        sum_c = fma(2.0 * J[2], cn, sum_c);
+#pragma unroll
+        for (int k = 0; k < 4; k++) st[k] = st[k + 1];
+    }
+    const double aa = -Amp * sum_a, bb = -Amp * sqrt(1 - e * e) * sum_b, cc = Amp * sum_c;
+    const double Aplus0 = -(1. + Ldotn2) * (aa * cos2gam - bb * sin2gam) + cc * (1 - Ldotn2);
+    const double Acros0 = 2. * Ldotn * (bb * cos2gam + aa * sin2gam);
+    const double Aplus = Aplus0 * rot[0] + Acros0 * rot[1];
+    const double Acros = Aplus0 * rot[2] + Acros0 * rot[3];
+    return make_double2(FplusI * Aplus + FcrosI * Acros, -(FplusII * Aplus + FcrosII * Acros));
 }
 
 // gpuAAK.cu:458-483: start index of every segment and the number of knots
@@ -458,19 +723,39 @@ __host__ __device__ inline int aak_plan(const double *h_t, int L, double dt, int
     return i < L ? i + 1 : L;
 }
 
+// aak_plan, one knot per lane: knots up to the first at or past the end.
 __global__ __launch_bounds__(64) void aak_plan_kernel(AakArgs a)
 {
-    if (threadIdx.x == 0) a.plan[a.L] = aak_plan(a.h_t, a.L, a.dt, a.out_len, a.plan);
+    const double T = (a.out_len - 1) * a.dt;
+    const int lane = threadIdx.x;
+    if (lane == 0) a.plan[0] = 0;
+    int count = a.L;
+    for (int base = 1; base < a.L; base += 64) {
+        const int i = base + lane;
+        const bool in = i < a.L;
+        const bool past = in && !(a.h_t[i] < T);
+        const unsigned long long end = __ballot(past);
+        const int first = end ? base + __ffsll(end) - 1 : a.L;
+        if (in && i < first) a.plan[i] = (int)ceil(a.h_t[i] / a.dt);
+        if (in && i == first) a.plan[i] = a.out_len;
+        if (end) {
+            count = first + 1;
+            break;
+        }
+    }
+    if (lane == 0) a.plan[a.L] = count;
 }
 
 #define AAK_THREADS 128
 
-// Three waves per SIMD (at most 168 registers, a few spills): the per-sample
-// Bessel recurrences and sincos chains are FP64-latency-bound, and the third
-// wave hides more of that than the spills cost (full year at 10 s, 30
-// harmonics: 7.1 ms against 8.2 ms at two waves; four waves, 7.5 ms).
+// What bounds it: FP64 VALU issue, ~600 instructions per harmonic (the two
+// recurrences of n + sqrt(40 n) steps) and ~1000 for the geometry of a sample.
+// Three waves per SIMD (168 registers, 48 spilled outside the recurrences): full
+// year at 10 s, 30 harmonics with the LISA response 1.40 ms, two waves 1.56 ms,
+// four 6.7 ms (6.64 ms with five recurrences per harmonic and the geometry
+// through its inverse functions).
 __global__ __launch_bounds__(AAK_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
-void aak_sum_kernel(AakArgs a)
+void aak_sum_kernel(AakArgs a, AakGeom geom)
 {
     const int npts = a.plan[a.L];
     const int nseg = npts - 1;
@@ -489,7 +774,7 @@ void aak_sum_kernel(AakArgs a)
     const long np = (long)(a.L - 1) * 6;
     for (int c = 0; c < 8; c++)
         for (int p = 0; p < 6; p++) sc[p][c] = a.interp[c * np + (long)j * 6 + p];
-    a.wave[i] = aak_sample(a, sc, a.h_t[j], a.h_t[j + 1] - a.h_t[j], i);
+    a.wave[i] = aak_sample_fast(a, geom, sc, a.h_t[j], a.h_t[j + 1] - a.h_t[j], i);
 }
 
 size_t aak_workspace_bytes(int init_len) { return sizeof(int) * (size_t)(init_len + 1); }
@@ -505,7 +790,8 @@ int launch_aak(AakArgs a, void *workspace, size_t workspace_bytes, hipStream_t s
     hipLaunchKernelGGL(aak_plan_kernel, dim3(1), dim3(64), 0, stream, a);
     FEW_HIP(hipGetLastError());
     const long blocks = ((long)a.out_len + AAK_THREADS - 1) / AAK_THREADS;
-    hipLaunchKernelGGL(aak_sum_kernel, dim3((unsigned)blocks), dim3(AAK_THREADS), 0, stream, a);
+    hipLaunchKernelGGL(aak_sum_kernel, dim3((unsigned)blocks), dim3(AAK_THREADS), 0, stream, a,
+                       aak_geom(a));
     FEW_HIP(hipGetLastError());
     return FEW_OK;
 }

@@ -490,4 +490,40 @@ void twin_fd_roots(const double *abcd, long n, double *out)
     }
 }
 
+// aak_bessel5 beside nr_jn5, orders order..order+4
+void twin_aak_bessel5(const int *order, const double *x, long n, double *fast, double *ref)
+{
+    for (long i = 0; i < n; i++) {
+        double f[5], r[5];
+        int st[5];
+        for (int k = 0; k < 5; k++) st[k] = nr_miller_start(order[i] + k >= 2 ? order[i] + k : 2);
+        aak_bessel5(order[i], x[i], st, f);
+        nr_jn5(order[i], x[i], r);
+        for (int k = 0; k < 5; k++) {
+            fast[5 * i + k] = f[k];
+            ref[5 * i + k] = r[k];
+        }
+    }
+}
+
+// twin_aak_waveform in the kernel's form (aak_sample_fast)
+int twin_aak_waveform_fast(double *wave, const double *interp, double M, double S, double mu,
+                           double qS, double phiS, double qK, double phiK, double dist, int nmodes,
+                           int mich, int L, int out_len, double dt, const double *h_t)
+{
+    AakArgs a{reinterpret_cast<double2 *>(wave), interp, h_t, M, S, mu, qS, phiS, qK, phiK, dist, dt,
+              nmodes, mich, L, out_len, nullptr};
+    std::vector<int> st(L + 1);
+    const int npts = aak_plan(h_t, L, dt, out_len, st.data());
+    const AakGeom g = aak_geom(a);
+    for (int j = 0; j + 1 < npts; j++) {
+        double sc[6][8];
+        for (int c = 0; c < 8; c++)
+            for (int p = 0; p < 6; p++) sc[p][c] = interp[((long)c * (L - 1) + j) * 6 + p];
+        for (int i = st[j]; i < st[j + 1]; i++)
+            a.wave[i] = aak_sample_fast(a, g, sc, h_t[j], h_t[j + 1] - h_t[j], i);
+    }
+    return 0;
+}
+
 }  // extern "C"
