@@ -3,14 +3,14 @@
 //
 // Mode-sum adjoint: one workgroup owns one chunk of one interval's samples
 // (at most `chunk` samples, never crossing an interval boundary) and one
-// group of ADJ_MODES modes, one mode per lane.  The chunk's sample state
-// (x, the three phases, g) is computed once per sample into LDS, then every
-// lane walks the staged samples and keeps its mode's twelve moments in
-// registers: sum x^p dL/dRe A, sum x^p dL/dIm A (p = 0..3) and
-// sum xp^p dL/dphi.  Nothing is reduced across lanes per sample; per chunk
-// the amplitude moments go to a partial buffer (chunk, 4, 2K) and the phase
-// moments (weighted by m, k, n) are reduced over the workgroup.  A second
-// kernel adds the chunks of each interval in a fixed order (deterministic).
+// group of ADJ_MODES cells (modes sharing (m, k, n)), one cell per lane.  Every
+// wave stages the state of its part of the samples (x, the three phases, g) and
+// walks them; a lane keeps its cell's twenty moments in registers: sum x^p
+// dL/d(P, Q, R, S) and sum xp^p dL/dphase, p = 0..3.  Nothing is reduced across
+// lanes per sample; per chunk the moments are expanded to the cells' modes in a
+// partial buffer (chunk, 4, 2K) and the phase moments (weighted by m, k, n) are
+// reduced over the workgroup.  A second kernel adds the chunks of each interval
+// in a fixed order (deterministic).
 #include <math.h>
 
 #include "adjoint.hpp"
@@ -20,8 +20,7 @@
 
 namespace few {
 
-#define ADJ_MODES 128   // lanes (modes) per workgroup
-#define ADJ_SUB 128     // samples staged in LDS per step
+#define ADJ_MODES 128   // cells per workgroup
 
 // Transposed spline build, in two parts.  Every system of one call shares
 // the knots, hence the matrix A^T of the not-a-knot system; LAPACK dgtsv's
@@ -391,132 +390,220 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-__global__ __launch_bounds__(ADJ_MODES) void adjoint_fp64_kernel(AdjArgs a)
-{
-    __shared__ double s_x[ADJ_SUB], s_pp[ADJ_SUB], s_pt[ADJ_SUB], s_pr[ADJ_SUB];
-    __shared__ double s_gr[ADJ_SUB], s_gi[ADJ_SUB], s_xp[ADJ_SUB];
-    __shared__ double s_red[ADJ_MODES / 64][12];
+// The moments of one cell over its samples: with h = (P cos + Q sin) +
+// i (R cos + S sin) (modesum_direct.hpp), G[p] holds sum x^p (g_re cos, g_re sin,
+// g_im cos, g_im sin) = dL/d(P, Q, R, S) of power p, and R[p] sum xp^p dL/dphase.
+struct CellMoments {
+    double G[4][4], R[4];
+};
 
-    const int c = blockIdx.x;
+// Wave-private staged samples
+struct AdjStage {
+    double x[64], Pp[64], Pt[64], Pr[64], gr[64], gi[64], xp[64];
+};
+
+// Samples [lo, hi) of interval j for the lane's cell (c, m, k, n); false if a
+// phase was outside sincos_half_turns' range (never, if BIG).
+template <bool BIG>
+__device__ __forceinline__ bool adj_cell_samples(const AdjArgs &a, int j, const Segment &sg, int lo,
+                                                 int hi, AdjStage &st, const double (&c)[4][4],
+                                                 double m, double k, double n, CellMoments &M)
+{
+    const int lane = threadIdx.x & 63;
+    const long np = (long)a.nseg * 3;
+    bool ok = true;
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        M.R[p] = 0.0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) M.G[p][e] = 0.0;
+    }
+    for (int base = lo; base < hi; base += 64) {
+        __builtin_amdgcn_wave_barrier();
+        {
+            const int i = base + lane;
+            double rp[8], rt[8], rr[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                rp[q] = a.pcoef[q * np + (long)j * 3 + 0];
+                rt[q] = a.pcoef[q * np + (long)j * 3 + 1];
+                rr[q] = a.pcoef[q * np + (long)j * 3 + 2];
+            }
+            SampleState s;
+            sample_state(a.dt, i, sg.h_t, sg.pt, sg.pw, rp, rt, rr, s);
+            const double2 g = i < hi ? a.grad[i] : make_double2(0.0, 0.0);
+            st.x[lane] = s.x;
+            st.Pp[lane] = s.Pp;
+            st.Pt[lane] = s.Pt;
+            st.Pr[lane] = s.Pr;
+            st.gr[lane] = g.x;
+            st.gi[lane] = g.y;
+            st.xp[lane] = a.dt * (double)i - sg.pt;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int cnt = min(64, hi - base);
+        for (int q = 0; q < cnt; q++) {
+            const double x = st.x[q], gr = st.gr[q], gi = st.gi[q], xp = st.xp[q];
+            const double phase = mode_phase(m, st.Pp[q], k, st.Pt[q], n, st.Pr[q]);
+            double sn, cs;
+            if (BIG) {
+                if (!sincos_cw(phase, sn, cs)) sincos(phase, &sn, &cs);
+            } else {
+                const bool in = sincos_half_turns(phase, sn, cs);
+                ok = ok && in;
+            }
+            const double x2 = x * x, x3 = x2 * x;
+            const double A[4] = {gr * cs, gr * sn, gi * cs, gi * sn};
+            double v[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                M.G[0][e] += A[e];
+                M.G[1][e] = fma(x, A[e], M.G[1][e]);
+                M.G[2][e] = fma(x2, A[e], M.G[2][e]);
+                M.G[3][e] = fma(x3, A[e], M.G[3][e]);
+                v[e] = fma(fma(fma(c[3][e], x, c[2][e]), x, c[1][e]), x, c[0][e]);
+            }
+            const double rho = fma(v[1], A[0], fma(-v[0], A[1], fma(v[3], A[2], -v[2] * A[3])));
+            const double xp2 = xp * xp, xp3 = xp2 * xp;
+            M.R[0] += rho;
+            M.R[1] = fma(xp, rho, M.R[1]);
+            M.R[2] = fma(xp2, rho, M.R[2]);
+            M.R[3] = fma(xp3, rho, M.R[3]);
+        }
+    }
+    return ok;
+}
+
+#define ADJ_PARTS 4     // waves sharing a workgroup's cells, a part of the chunk each
+
+// One workgroup: a chunk of one interval's samples and ADJ_MODES cells (modes
+// sharing (m, k, n), cells.hpp), one per lane.  ADJ_PARTS waves hold the same
+// cells and a part of the samples each; their moments are added in LDS and
+// expanded to the cells' modes, so the chunk's record is per mode as before.
+//
+// What bounds it: FP64 VALU issue, ~80 instructions per (cell, sample).  One
+// month, 500 modes (366 cells): 0.476 ms; one year, 3843 modes: 6.4 ms (1.07 and
+// 39.3 ms with one lane per mode and two waves per workgroup).  Four waves per
+// SIMD with 46 spilled registers; without the spills (three waves) 0.51 and
+// 7.2 ms.
+__global__ __launch_bounds__(64 * ADJ_PARTS * (ADJ_MODES / 64), 4) void adjoint_fp64_kernel(AdjArgs a)
+{
+    constexpr int HALVES = ADJ_MODES / 64, VALS = 20;
+    __shared__ union {
+        AdjStage stage[ADJ_PARTS * HALVES];
+        double sum[2][VALS][ADJ_MODES];   // two parts at a time
+    } sh;
+    __shared__ double s_red[HALVES][12];
+    const int b = blockIdx.x;
     const int total = a.prefix[a.nseg];
-    if (c >= total) return;  // uniform over the workgroup
+    const int ncell = a.cells.start ? *a.cells.count : a.K;
+    if (b >= total || (int)blockIdx.y * ADJ_MODES >= ncell) return;  // uniform over the workgroup
     int lo_s = 0, hi_s = a.nseg;
     while (hi_s - lo_s > 1) {
         const int mid = (lo_s + hi_s) >> 1;
-        if (a.prefix[mid] <= c) lo_s = mid; else hi_s = mid;
+        if (a.prefix[mid] <= b) lo_s = mid; else hi_s = mid;
     }
     const int j = lo_s;
     const Segment sg = a.segs[j];
-    const int lo = sg.start + (c - a.prefix[j]) * a.chunk;
+    const int lo = sg.start + (b - a.prefix[j]) * a.chunk;
     const int hi = min(lo + a.chunk, sg.end);
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = wv % HALVES, part = wv / HALVES;
     const int K = a.K;
-    const int mode = blockIdx.y * ADJ_MODES + tid;
-    const bool act = mode < K;
-
-    double cr0 = 0, cr1 = 0, cr2 = 0, cr3 = 0, ci0 = 0, ci1 = 0, ci2 = 0, ci3 = 0;
-    double ypr = 0, ypi = 0, ymr = 0, ymi = 0, mm = 0, kk = 0, nn = 0;
+    const int cell = blockIdx.y * ADJ_MODES + half * 64 + lane;
+    const bool act = cell < ncell;
+    int s0 = cell, s1 = cell;
     if (act) {
-        const long nb = (long)a.L * 2 * K;
-        const long br = (long)j * 2 * K + mode, bi = br + K;
-        cr0 = a.interp[br]; cr1 = a.interp[nb + br]; cr2 = a.interp[2 * nb + br]; cr3 = a.interp[3 * nb + br];
-        ci0 = a.interp[bi]; ci1 = a.interp[nb + bi]; ci2 = a.interp[2 * nb + bi]; ci3 = a.interp[3 * nb + bi];
-        const double2 yp = a.ylm[mode];
-        ypr = yp.x;
-        ypi = yp.y;
-        const int m = a.m[mode];
-        if (m != 0) {
-            const double2 ym = a.ylm[K + mode];
-            ymr = ym.x;
-            ymi = ym.y;
-        }
-        mm = (double)m;
-        kk = (double)a.k[mode];
-        nn = (double)a.n[mode];
+        s0 = a.cells.start ? a.cells.start[cell] : cell;
+        s1 = a.cells.start ? a.cells.start[cell + 1] : cell + 1;
     }
-    const long np = (long)a.nseg * 3;
-    double rp[8], rt[8], rr[8];
+    const long nb = (long)a.L * 2 * K;
+    const double *ip = a.interp + (long)j * 2 * K;
+    double c[4][4], mm = 0.0, kk = 0.0, nn = 0.0;
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-        rp[q] = a.pcoef[q * np + (long)j * 3 + 0];
-        rt[q] = a.pcoef[q * np + (long)j * 3 + 1];
-        rr[q] = a.pcoef[q * np + (long)j * 3 + 2];
+    for (int p = 0; p < 4; p++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) c[p][e] = 0.0;
+    for (int s = s0; s < s1; s++) {
+        const int mode = a.cells.start ? a.cells.member[s] : s;
+        if (s == s0) {
+            mm = (double)a.m[mode];
+            kk = (double)a.k[mode];
+            nn = (double)a.n[mode];
+        }
+        const double2 yp = a.ylm[mode], ym = a.ylm[K + mode];
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+            cell_coef_add(ip[p * nb + mode], ip[p * nb + K + mode], yp.x, yp.y, ym.x, ym.y,
+                          mm != 0.0, c[p]);
     }
-
-    double dr0 = 0, dr1 = 0, dr2 = 0, dr3 = 0, di0 = 0, di1 = 0, di2 = 0, di3 = 0;
-    double R0 = 0, R1 = 0, R2 = 0, R3 = 0;
-    for (int base = lo; base < hi; base += ADJ_SUB) {
+    // this wave's part of the chunk, in whole groups of 64 samples
+    const int per = ((hi - lo + 64 * ADJ_PARTS - 1) / (64 * ADJ_PARTS)) * 64;
+    const int plo = min(hi, lo + part * per), phi = min(hi, plo + per);
+    CellMoments M;
+    const bool ok = adj_cell_samples<false>(a, j, sg, plo, phi, sh.stage[wv], c, mm, kk, nn, M);
+    // phases beyond 1e8 rad (or NaN): again with the library's sincos
+    if (__any(act && !ok)) adj_cell_samples<true>(a, j, sg, plo, phi, sh.stage[wv], c, mm, kk, nn, M);
+    // parts 2, 3 into 0, 1, then 1 into 0
+    const int col = half * 64 + lane;
+#pragma unroll
+    for (int step = ADJ_PARTS / 2; step >= 1; step /= 2) {
         __syncthreads();
-        {
-            const int i = base + tid;
-            SampleState st;
-            sample_state(a.dt, i, sg.h_t, sg.pt, sg.pw, rp, rt, rr, st);
-            double gr = 0.0, gi = 0.0;
-            if (i < hi) {
-                const double2 g = a.grad[i];
-                gr = g.x;
-                gi = g.y;
-            }
-            s_x[tid] = st.x;
-            s_pp[tid] = st.Pp;
-            s_pt[tid] = st.Pt;
-            s_pr[tid] = st.Pr;
-            s_gr[tid] = gr;
-            s_gi[tid] = gi;
-            s_xp[tid] = a.dt * (double)i - sg.pt;
+        if (part >= step && part < 2 * step) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) sh.sum[part - step][i][col] = M.G[i / 4][i % 4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) sh.sum[part - step][16 + i][col] = M.R[i];
         }
         __syncthreads();
-        const int cnt = min(ADJ_SUB, hi - base);
-        for (int q = 0; q < cnt; q++) {
-            const double x = s_x[q];
-            const double phase = mode_phase(mm, s_pp[q], kk, s_pt[q], nn, s_pr[q]);
-            double e_im, e_re;
-            if (!sincos_cw(-phase, e_im, e_re)) sincos(-phase, &e_im, &e_re);
-            const double gr = s_gr[q], gi = s_gi[q];
-            // q+ = conj(g) e, q- = conj(g) conj(e)
-            const double A1 = gr * e_re, A2 = gi * e_im, A3 = gr * e_im, A4 = gi * e_re;
-            const double qpr = A1 + A2, qpi = A3 - A4, qmr = A1 - A2, qmi = -(A3 + A4);
-            const double Wr = qpr * ypr - qpi * ypi, Wi = qpr * ypi + qpi * ypr;
-            const double Vr = qmr * ymr - qmi * ymi, Vi = qmr * ymi + qmi * ymr;
-            const double d_re = Wr + Vr, d_im = Vi - Wi;
-            const double a_re = cr0 + x * (cr1 + x * (cr2 + x * cr3));
-            const double a_im = ci0 + x * (ci1 + x * (ci2 + x * ci3));
-            const double rho = a_im * d_re - a_re * d_im;
-            const double x2 = x * x, x3 = x2 * x;
-            dr0 += d_re; dr1 += x * d_re; dr2 += x2 * d_re; dr3 += x3 * d_re;
-            di0 += d_im; di1 += x * d_im; di2 += x2 * d_im; di3 += x3 * d_im;
-            const double xp = s_xp[q], xp2 = xp * xp, xp3 = xp2 * xp;
-            R0 += rho; R1 += xp * rho; R2 += xp2 * rho; R3 += xp3 * rho;
+        if (part < step) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) M.G[i / 4][i % 4] += sh.sum[part][i][col];
+#pragma unroll
+            for (int i = 0; i < 4; i++) M.R[i] += sh.sum[part][16 + i][col];
         }
     }
-    if (act) {
+    if (part == 0) {
         const long K2 = 2L * K;
-        double *pa = a.part_amp + (long)c * 4 * K2;
-        pa[mode] = dr0;          pa[K + mode] = di0;
-        pa[K2 + mode] = dr1;     pa[K2 + K + mode] = di1;
-        pa[2 * K2 + mode] = dr2; pa[2 * K2 + K + mode] = di2;
-        pa[3 * K2 + mode] = dr3; pa[3 * K2 + K + mode] = di3;
-    }
-    // phase moments: sum over the group's modes of (m, k, n) * R_p, [p][q] order
-    const double Rs[4] = {R0, R1, R2, R3};
-    const int wv = tid >> 6, lane = tid & 63;
+        double *pa = a.part_amp + (long)b * 4 * K2;
+        for (int s = s0; s < s1; s++) {
+            const int mode = a.cells.start ? a.cells.member[s] : s;
+            const double2 yp = a.ylm[mode], ym = a.ylm[K + mode];
 #pragma unroll
-    for (int p = 0; p < 4; p++) {
-        const double vm = wave_sum(mm * Rs[p]);
-        const double vk = wave_sum(kk * Rs[p]);
-        const double vn = wave_sum(nn * Rs[p]);
-        if (lane == 0) {
-            s_red[wv][p * 3 + 0] = vm;
-            s_red[wv][p * 3 + 1] = vk;
-            s_red[wv][p * 3 + 2] = vn;
+            for (int p = 0; p < 4; p++) {
+                // dL/d(Re C+, Im C+, Re C-, Im C-), then the member's A
+                const double pr = M.G[p][0] - M.G[p][3], pi = M.G[p][1] + M.G[p][2];
+                double d_re = yp.x * pr + yp.y * pi, d_im = yp.x * pi - yp.y * pr;
+                if (mm != 0.0) {
+                    const double mr = M.G[p][0] + M.G[p][3], mi = M.G[p][2] - M.G[p][1];
+                    d_re += ym.x * mr + ym.y * mi;
+                    d_im += ym.y * mr - ym.x * mi;
+                }
+                pa[p * K2 + mode] = d_re;
+                pa[p * K2 + K + mode] = d_im;
+            }
+        }
+        // phase moments: sum over the group's cells of (m, k, n) * R_p, [p][q] order
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const double vm = wave_sum(mm * M.R[p]);
+            const double vk = wave_sum(kk * M.R[p]);
+            const double vn = wave_sum(nn * M.R[p]);
+            if (lane == 0) {
+                s_red[half][p * 3 + 0] = vm;
+                s_red[half][p * 3 + 1] = vk;
+                s_red[half][p * 3 + 2] = vn;
+            }
         }
     }
     __syncthreads();
     if (tid < 12) {
-        double v = 0.0;
+        double sum = 0.0;
 #pragma unroll
-        for (int w = 0; w < ADJ_MODES / 64; w++) v += s_red[w][tid];
-        a.part_phase[((long)c * a.groups + blockIdx.y) * 12 + tid] = v;
+        for (int w = 0; w < HALVES; w++) sum += s_red[w][tid];
+        a.part_phase[((long)b * a.groups + blockIdx.y) * 12 + tid] = sum;
     }
 }
 
@@ -545,29 +632,21 @@ __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjReduceArgs r)
     if (blockIdx.x == 0 && threadIdx.x < 12) {
         const int v = threadIdx.x;
         double acc = 0.0;
+        // groups past the cells wrote nothing
+        const int ncell = r.cells.start ? *r.cells.count : r.K;
+        const int groups = min(r.groups, (ncell + ADJ_MODES - 1) / ADJ_MODES);
         for (int c = c0; c < c1; c++)
-            for (int g = 0; g < r.groups; g++) acc += r.part_phase[((long)c * r.groups + g) * 12 + v];
+            for (int g = 0; g < groups; g++) acc += r.part_phase[((long)c * r.groups + g) * 12 + v];
         const int p = v / 3, q = v % 3;
         r.g_phase[((long)p * r.L + j) * 3 + q] = acc;
     }
 }
 
-size_t adjoint_workspace_bytes(int L, int out_len, int K, int chunk, int groups)
-{
-    const long max_chunks = (long)(out_len + chunk - 1) / chunk + L;
-    size_t b = 0;
-    b += ((sizeof(Segment) * (size_t)L + 255) / 256) * 256;
-    b += ((sizeof(int) * (size_t)(L + 1) + 255) / 256) * 256;
-    b += ((sizeof(double) * (size_t)max_chunks * 8 * K + 255) / 256) * 256;
-    b += ((sizeof(double) * (size_t)max_chunks * groups * 12 + 255) / 256) * 256;
-    return b;
-}
-
 int launch_adjoint_fp64(const AdjArgs &a, int max_chunks, hipStream_t stream)
 {
     if (max_chunks <= 0 || a.K <= 0) return FEW_OK;
-    hipLaunchKernelGGL(adjoint_fp64_kernel, dim3(max_chunks, a.groups), dim3(ADJ_MODES), 0, stream,
-                       a);
+    hipLaunchKernelGGL(adjoint_fp64_kernel, dim3(max_chunks, a.groups),
+                       dim3(ADJ_MODES * ADJ_PARTS), 0, stream, a);
     FEW_HIP(hipGetLastError());
     return FEW_OK;
 }

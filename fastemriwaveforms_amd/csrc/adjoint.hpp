@@ -18,6 +18,7 @@
 // A^T lambda = dL/dz, then fill_B transposed.
 #pragma once
 
+#include "cells.hpp"
 #include "few_common.hpp"
 #include "modesum_fact.hpp"
 
@@ -34,7 +35,8 @@ struct AdjArgs {
     int nseg, L, K;
     double dt;
     int chunk;                // samples per chunk
-    int groups;               // mode groups (blockIdx.y)
+    int groups;               // cell groups (blockIdx.y), for one cell per mode
+    CellIndex cells;          // modes sharing (m, k, n)
     double *part_amp;         // (max_chunks, 4, 2K) per-chunk partial dL/dc
     double *part_phase;       // (max_chunks, groups, 12) per-chunk partial phase moments
 };
@@ -44,6 +46,7 @@ struct AdjReduceArgs {
     const double *part_amp;
     const double *part_phase;
     int nseg, L, K, groups;
+    CellIndex cells;
     double *g_interp;         // (4, L, 2K) out
     double *g_phase;          // (4, L, 3) out
 };
@@ -129,7 +132,6 @@ int launch_adjoint16(const Adj16Args &a, int max_chunks, hipStream_t stream);
 int launch_adjoint16_finish(const Adj16Args &a, const Adj16FinishArgs &f, hipStream_t stream,
                             bool reduce_chunks);
 
-size_t adjoint_workspace_bytes(int L, int out_len, int K, int chunk, int groups);
 int launch_adjoint_fp64(const AdjArgs &a, int max_chunks, hipStream_t stream);
 int launch_adjoint_reduce(const AdjReduceArgs &r, hipStream_t stream);
 int launch_spline_adjoint(const SplineAdjArgs &a, hipStream_t stream);

@@ -437,7 +437,7 @@ static int run_waveform(double2 *wave, const double *interp, const double *pt, c
 // ------------------------------------------------------------------ adjoint
 
 #define ADJ_CHUNK 2048   // samples per chunk of the mode-sum adjoint
-#define ADJ_GROUP 128    // modes per workgroup of the mode-sum adjoint
+#define ADJ_GROUP 128    // cells per workgroup of the mode-sum adjoint
 
 struct AdjLayout {
     size_t segs, prefix, amp, phase, total;
@@ -792,7 +792,7 @@ size_t few_adjoint_workspace_bytes(int init_len, int out_len, int num_modes, int
 {
     (void)precision;
     if (init_len < 2 || out_len < 0 || num_modes < 0) return 0;
-    return adj_layout(init_len, out_len, num_modes).total;
+    return adj_layout(init_len, out_len, num_modes).total + cell_index_bytes(num_modes);
 }
 
 int few_waveform_adjoint_async(const void *grad_wave, const double *interp_array,
@@ -849,6 +849,9 @@ int few_waveform_adjoint_async(const void *grad_wave, const double *interp_array
     a.part_amp = reinterpret_cast<double *>(ws + al.amp);
     a.part_phase = reinterpret_cast<double *>(ws + al.phase);
     if (K > 0 && out_len > 0) {
+        // behind the parts every call needs (a workspace without it: ungrouped)
+        rc = group_modes(d_m, d_k, d_n, K, ws, workspace_bytes, al.total, a.cells, st);
+        if (rc) return rc;
         rc = launch_adjoint_fp64(a, (int)al.max_chunks, st);
         if (rc) return rc;
     }
@@ -859,6 +862,7 @@ int few_waveform_adjoint_async(const void *grad_wave, const double *interp_array
     r.nseg = L - 1;
     r.L = L;
     r.K = K;
+    r.cells = a.cells;
     r.groups = (K > 0 && out_len > 0) ? al.groups : 0;
     r.g_interp = g_interp;
     r.g_phase = g_phase;
@@ -871,8 +875,8 @@ size_t few_plan_adjoint_workspace_bytes(const void *plan, int init_len, int out_
 {
     if (init_len < 2 || out_len < 0) return 0;
     if ((precision != FEW_PRECISION_MIXED16 && precision != FEW_PRECISION_FACT64) || !plan)
-        return adj_layout(init_len, out_len, plan ? static_cast<const FactPlan *>(plan)->host.K : 0)
-            .total;
+        return few_adjoint_workspace_bytes(
+            init_len, out_len, plan ? static_cast<const FactPlan *>(plan)->host.K : 0, precision);
     const FactPlanHost &h = static_cast<const FactPlan *>(plan)->host;
     return (precision == FEW_PRECISION_FACT64 ? adj64_layout(h, init_len, out_len)
                                               : adj16_layout(h, init_len, out_len)).total;

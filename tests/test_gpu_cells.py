@@ -103,3 +103,72 @@ def test_phases_beyond_the_fast_range(gpu):
     inp = dataclasses.replace(inp, dense=dense)
     h, ref = _run(inp), oracle_waveform(inp)
     assert oracle.rel_l2(h, ref) <= TOL
+
+
+# ------------------------------------------------------------------ adjoint
+
+def _adjoint(inp, g, ws_bytes=None):
+    """(dL/d amplitude coefficients (4, L, 2K), dL/d phase coefficients (4, L, 3))"""
+    import torch
+    from fastemriwaveforms_amd._lib import check, lib
+    from fastemriwaveforms_amd.pipeline import ModeSumProblem, _stream
+    p = ModeSumProblem(inp)
+    p.build_splines()
+    need = int(lib().few_adjoint_workspace_bytes(p.L, p.N, p.K, 0))
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    gi = torch.full((4, p.L, 2 * p.K), 5.0, dtype=torch.float64, device="cuda")
+    gp = torch.full((4, p.L, 3), 5.0, dtype=torch.float64, device="cuda")
+    gd = torch.from_numpy(g).cuda()
+    check(lib().few_waveform_adjoint_async(
+        gd.data_ptr(), p.interp.data_ptr(), p.t.data_ptr(), p.pcoef.data_ptr(), p.m.data_ptr(),
+        p.k.data_ptr(), p.n.data_ptr(), p.L, p.N, p.K, p.ylm.data_ptr(), p.dt, p.t.data_ptr(),
+        gi.data_ptr(), gp.data_ptr(), 0, ws.data_ptr(), need if ws_bytes is None else ws_bytes(need, p),
+        _stream()), "adjoint")
+    return gi.cpu().numpy(), gp.cpu().numpy()
+
+
+def _adjoint_ref(inp, g):
+    from helpers import oracle_coefficients
+    interp, pcoef = oracle_coefficients(inp)
+    return oracle.waveform_adjoint(g, interp, inp.t, pcoef, inp.m, inp.k, inp.n, inp.L, inp.num_pts,
+                                   inp.K, inp.ylms, inp.dt, inp.t)
+
+
+def _close(got, ref):
+    # per power: each is a sum of its own scale
+    for p in range(4):
+        assert oracle.rel_l2(got[0][p], ref[0][p]) <= TOL
+        assert oracle.rel_l2(got[1][p], ref[1][p]) <= 10 * TOL   # cancelling sums over all modes
+
+
+@pytest.mark.parametrize("K", [1, 63, 64, 65, 127, 128, 129, 400, 1500])
+def test_adjoint_mode_counts(gpu, K):
+    inp = _input(K, 500 + K, L=6)
+    rng = np.random.default_rng(K)
+    g = rng.normal(size=inp.num_pts) + 1j * rng.normal(size=inp.num_pts)
+    _close(_adjoint(inp, g), _adjoint_ref(inp, g))
+
+
+@pytest.mark.parametrize("samples", [1, 63, 64, 65, 255, 257, 2048, 2049, 4500])
+def test_adjoint_interval_lengths(gpu, samples):
+    """Intervals of every length around the 64-sample groups and the chunk."""
+    inp = _input(70, 21, T=0.004, L=5)
+    t = np.array([0.0, samples, samples + 700, samples + 701, 12000]) * inp.dt
+    inp = dataclasses.replace(inp, t=t, num_pts=samples + 2000)
+    rng = np.random.default_rng(samples)
+    g = rng.normal(size=inp.num_pts) + 1j * rng.normal(size=inp.num_pts)
+    _close(_adjoint(inp, g), _adjoint_ref(inp, g))
+
+
+def test_adjoint_ungrouped_and_big_phases(gpu):
+    inp = _input(90, 33, L=6)
+    rng = np.random.default_rng(0)
+    g = rng.normal(size=inp.num_pts) + 1j * rng.normal(size=inp.num_pts)
+    ref = _adjoint_ref(inp, g)
+    _close(_adjoint(inp, g), ref)
+    # one byte short of the index's room: one cell per mode
+    _close(_adjoint(inp, g, ws_bytes=lambda need, p: need - 1), ref)
+    dense = inp.dense.copy()
+    dense[0, 2:4] += 3.0e8
+    inp = dataclasses.replace(inp, dense=dense)
+    _close(_adjoint(inp, g), _adjoint_ref(inp, g))
