@@ -28,7 +28,12 @@ namespace few {
 
 #define SPLINE_MAX_GROUPS 4
 #define SPLINE_PF 8  // prefetch distance (steps) of the sequential sweeps
-#define SPLINE_SHARED_MAX_L 150  // LDS path: (2 * 32 + 6) * L doubles per 32-system block
+// LDS path: (2 * 32 + 6) * L doubles per 32-system block, 290 knots in 160 KiB.
+// Above 146 knots a CU holds one block instead of two, which still wins where
+// there is more than a block per CU: 7686 systems of 151 / 200 knots take 70 /
+// 90 us (134 / 175 us with a lane per system and its scratch in HBM), 30000 of
+// 200 / 290 knots 338 / 485 us (366 / 534).
+#define SPLINE_SHARED_MAX_L 290
 #define SPLINE_TILE_BATCH 24     // knot-value loads in flight per lane while staging a tile
 
 struct SplineArgs {
