@@ -30,9 +30,9 @@ namespace few {
 #define SPLINE_PF 8  // prefetch distance (steps) of the sequential sweeps
 // LDS path: (2 * 32 + 6) * L doubles per 32-system block, 290 knots in 160 KiB.
 // Above 146 knots a CU holds one block instead of two, which still wins where
-// there is more than a block per CU: 7686 systems of 151 / 200 knots take 70 /
-// 90 us (134 / 175 us with a lane per system and its scratch in HBM), 30000 of
-// 200 / 290 knots 338 / 485 us (366 / 534).
+// there is more than a block per CU: 7686 systems of 151 / 200 knots take 62 /
+// 80 us (134 / 175 us with a lane per system and its scratch in HBM), 30000 of
+// 290 knots 397 us (534).
 #define SPLINE_SHARED_MAX_L 290
 #define SPLINE_TILE_BATCH 24     // knot-value loads in flight per lane while staging a tile
 
@@ -522,17 +522,39 @@ __host__ __device__ void spline_one_system(const SplineArgs &a, int gi, int s)
 #define SPLINE_BLOCK 256  // threads of the shared-knot block (4 waves)
 #define SPLINE_SPB 32     // systems per shared-knot block (half a wave)
 
+// Progress counters of a shared-knot block (LDS), one writer each; the readers
+// spin on them, and every writer runs to its end whatever the readers do.
+__device__ __forceinline__ void spline_post(int *c, int v)
+{
+    __hip_atomic_store(c, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ int spline_peek(int *c)
+{
+    return __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(c, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+
 // A block of SPLINE_SPB systems of a group on shared knots, four waves; the
 // two halves of a wave take alternate knots / rows / intervals of the same
 // systems.  Work that is parallel over (system, knot) is spread over the
-// waves; only what is sequential along the knots runs on a single wave:
+// waves; only what is sequential along the knots runs on a single wave, and
+// the chains follow each other at a distance of a few rows instead of one
+// after the other:
 //   wave 3:     the shared matrix (prep_row's rows, one per lane), then
 //               dgtsv's elimination chain (every lane the same chain);
 //   waves 0-2:  meanwhile each stages the knot values of a third of the rows
 //               (plus the neighbouring knots those rows read) and forms
 //               their right-hand sides, reading only what it staged itself;
-//   wave 0:     every system's sweeps (one lane per system) out of LDS;
-//   waves 0-3:  the coefficients of the intervals and their stores.
+//   wave 0:     every system's forward sweep (one lane per system) out of LDS,
+//               behind the elimination; then the back substitution, with
+//               reciprocals of the diagonal (dgtsv_back);
+//   waves 1-3:  the coefficients of the intervals and their stores, behind the
+//               back substitution.
+// What bounds it: the latency of those chains, one dependent FP64 operation after
+// another.  7686 systems of 120 knots: 50 us; 30000 of 290 knots: 397 us (57
+// and 485 us with the chains, 18 us for the elimination and 21 us for the sweeps,
+// and the coefficients one after the other, and a division per step of the back
+// substitution).
 __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double *lds)
 {
     constexpr int S = SPLINE_SPB;
@@ -542,10 +564,15 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
     const int lane = tid & 63, wv = tid >> 6;
     const int half = lane / S, ls = lane % S;
     double *sx = lds, *F = sx + n, *sy = F + 5 * n, *sb = sy + (long)n * S;
-    __shared__ int s_info;
+    // rows eliminated, waves whose right-hand sides are in place, lowest solved row
+    __shared__ int s_info, s_elim, s_rhs[2], s_solved;
     const int s0 = blk * S;
     const int nloc = min(S, G.nsys - s0);
     for (int i = tid; i < n; i += SPLINE_BLOCK) sx[i] = G.t[(long)i * G.t_knot];
+    if (tid == 0) {
+        s_elim = s_rhs[0] = s_rhs[1] = 0;
+        s_solved = n;
+    }
     __syncthreads();
     if (wv == 3) {
         double *piv = F, *fact = F + n, *d = F + 2 * n, *du = F + 3 * n, *dl = F + 4 * n;
@@ -561,8 +588,10 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
         // (identical on every lane: identical stores, no divergence)
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        const int info = dgtsv_factor_ahead<8>(n, d, du, dl, piv, fact);
+        const int info = dgtsv_factor_ahead<8>(n, d, du, dl, piv, fact,
+                                               [&](int i) { spline_post(&s_elim, i); });
         if (lane == 0) s_info = info;
+        spline_post(&s_elim, n);
     } else {
         const int c = (n + 2) / 3;
         const int r0 = wv * c, r1 = min(n, r0 + c);
@@ -594,25 +623,47 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
             }
         }
     }
+    if (wv == 1 || wv == 2) spline_post(&s_rhs[wv - 1], 1);
+    if (wv == 0) {
+        while (!spline_peek(&s_rhs[0]) || !spline_peek(&s_rhs[1])) __builtin_amdgcn_s_sleep(1);
+        // after an early return of the elimination this sweeps over rows that
+        // mean nothing; the systems are then done one by one below
+        if (half == 0)
+            dgtsv_forward(n, F, sb + ls, S, [&](int i) {
+                while (spline_peek(&s_elim) < i) __builtin_amdgcn_s_sleep(1);
+            });
+    }
     __syncthreads();
     if (s_info != 0) {  // singular: dgtsv's early return, handled system by system
         if (wv == 0 && half == 0) spline_one_system(a, gi, s0 + ls);
         return;
     }
-    if (wv == 0 && half == 0) dgtsv_sweeps(n, F, sb + ls, S);
-    __syncthreads();
+    if (wv == 0) {
+        // the reciprocals over the elimination's factors, which are spent
+        double *rec = F + n;
+        const double *d = F + 2 * n;
+        for (int r = lane; r < n; r += 64) rec[r] = 1.0 / d[r];
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (half == 0)
+            dgtsv_back(n, F, rec, sb + ls, S, [&](int i) { spline_post(&s_solved, i); });
+        spline_post(&s_solved, 0);
+        return;
+    }
     if (ls >= nloc) return;
-    // coefficients of interval i on lane group i % 8 (wave, half); the group
-    // holding interval n - 2 also writes the final derivatives
-    // (fill_final_derivs, interpolate.cu:242-280)
-    const int grp = 2 * wv + half;
+    // coefficients: from the last interval down, two at a time per wave (1-3).
+    // The first half also writes the final derivatives (fill_final_derivs,
+    // interpolate.cu:242-280).
     const int s = s0 + ls;
     double c1L = 0.0, c2L = 0.0, c3L = 0.0;
-#pragma unroll 2
-    for (int i = grp; i < n - 1; i += 8)
-        spline_emit(G, s, n, i, sb[(long)i * S + ls], sb[(long)(i + 1) * S + ls], sx[i], sx[i + 1],
-                    sy[(long)i * S + ls], sy[(long)(i + 1) * S + ls], c1L, c2L, c3L);
-    if (!G.dense && grp == (n - 2) % 8) {
+    for (int top = n - 2 - 2 * (wv - 1); top >= 0; top -= 6) {
+        while (spline_peek(&s_solved) > max(top - 1, 0)) __builtin_amdgcn_s_sleep(1);
+        const int i = top - half;
+        if (i >= 0)
+            spline_emit(G, s, n, i, sb[(long)i * S + ls], sb[(long)(i + 1) * S + ls], sx[i], sx[i + 1],
+                        sy[(long)i * S + ls], sy[(long)(i + 1) * S + ls], c1L, c2L, c3L);
+    }
+    if (!G.dense && wv == 1 && half == 0) {
         const double xx = sx[n - 1] - sx[n - 2];
         const double x2 = xx * xx;
         double *out = G.out;

@@ -87,9 +87,14 @@ __host__ __device__ inline int dgtsv_factor(int n, double *d, double *du, double
 // and each step's two pivot branches as selects around one division: for a
 // matrix in LDS, one wait per PF steps and no branch per step on the chain.
 // Same operations on the same operands, same results and early returns.
-template <int PF>
+// done(i): called as the chain goes, steps below i are recorded.
+struct DgtsvNoHook {
+    __host__ __device__ void operator()(int) const {}
+};
+
+template <int PF, class Done = DgtsvNoHook>
 __host__ __device__ inline int dgtsv_factor_ahead(int n, double *d, double *du, double *dl,
-                                                  double *piv, double *fact)
+                                                  double *piv, double *fact, Done done = Done())
 {
 #pragma clang fp contract(off)
     double di = d[0], dui = n > 1 ? du[0] : 0.0;
@@ -126,6 +131,7 @@ __host__ __device__ inline int dgtsv_factor_ahead(int n, double *d, double *du, 
                 di = dnew;
             }
         }
+        done(i0 + PF < n - 2 ? i0 + PF : n - 2);
     }
     if (n > 1) {
         const int i = n - 2;
@@ -160,18 +166,21 @@ __host__ __device__ inline int dgtsv_factor_ahead(int n, double *d, double *du, 
 #define DGTSV_SWEEP_PF 8  // values fetched ahead of the sweep recurrences
 
 // dgtsv's forward sweep of one right-hand side b (stride bs) with the
-// elimination F = piv | fact | d | du | dl recorded by dgtsv_factor, then the
-// back substitution: the solution into b.  dgtsv's operations in its order;
-// the operands of the next DGTSV_SWEEP_PF steps are read before the dependent
-// arithmetic and each pivot choice is a select (no branch on the chain).
-__host__ __device__ inline void dgtsv_sweeps(int n, const double *F, double *bv, long bs)
+// elimination F = piv | fact | d | du | dl recorded by dgtsv_factor: b is
+// left as the upper triangle's right-hand side.  dgtsv's operations in its
+// order; the operands of the next DGTSV_SWEEP_PF steps are read before the
+// dependent arithmetic and each pivot choice is a select (no branch on the
+// chain).  wait(i): called before the records of the steps below i are read.
+template <class Wait>
+__host__ __device__ inline void dgtsv_forward(int n, const double *F, double *bv, long bs, Wait wait)
 {
 #pragma clang fp contract(off)
 #define SB(i) bv[(long)(i) * bs]
-    const double *piv = F, *fact = F + n, *d = F + 2 * n, *du = F + 3 * n, *dl = F + 4 * n;
+    const double *piv = F, *fact = F + n;
     double cur = SB(0);
     for (int i0 = 0; i0 < n - 1; i0 += DGTSV_SWEEP_PF) {
         double nbv[DGTSV_SWEEP_PF], fv[DGTSV_SWEEP_PF], pv[DGTSV_SWEEP_PF];
+        wait(i0 + DGTSV_SWEEP_PF < n - 1 ? i0 + DGTSV_SWEEP_PF : n - 1);
 #pragma unroll
         for (int u = 0; u < DGTSV_SWEEP_PF; u++) {
             const int i = i0 + u < n - 2 ? i0 + u : n - 2;
@@ -192,7 +201,42 @@ __host__ __device__ inline void dgtsv_sweeps(int n, const double *F, double *bv,
             }
         }
     }
-    double x_next = cur / d[n - 1];
+    SB(n - 1) = cur;
+}
+
+// a / d given r = 1 / d, both correctly rounded: the quotient is refined by its
+// exact remainder twice (the first makes it faithful, the second then rounds it
+// correctly: P. Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", 1990).  Five dependent operations where the division
+// takes about twelve; valid while no remainder underflows, which div_in_range
+// of a and d (and a != 0, whose sign the remainders would lose) ensures.
+__host__ __device__ inline double div_by_reciprocal(double a, double d, double r)
+{
+    double q = a * r;
+    q = fma(fma(-q, d, a), r, q);
+    return fma(fma(-q, d, a), r, q);
+}
+
+// |x| in [2^-400, 2^400)
+__host__ __device__ inline bool div_in_range(double x)
+{
+    unsigned long long b;
+    __builtin_memcpy(&b, &x, 8);
+    return (((unsigned)(b >> 52) & 0x7ffu) - 623u) < 800u;
+}
+
+// dgtsv's back substitution (the solution into b).  rec: the reciprocals of the
+// diagonal, taken in place of the divisions with the same results (the steps
+// of a group are repeated with divisions where a value is out of
+// div_by_reciprocal's range); null: divisions.  done(i): called as the chain goes,
+// the solution is in place from i on.
+template <class Done>
+__host__ __device__ inline void dgtsv_back(int n, const double *F, const double *rec, double *bv,
+                                           long bs, Done done)
+{
+#pragma clang fp contract(off)
+    const double *d = F + 2 * n, *du = F + 3 * n, *dl = F + 4 * n;
+    double x_next = SB(n - 1) / d[n - 1];
     SB(n - 1) = x_next;
     // row n - 2 has no second super-diagonal term
     double x_next2 = x_next;
@@ -200,6 +244,7 @@ __host__ __device__ inline void dgtsv_sweeps(int n, const double *F, double *bv,
     SB(n - 2) = x_next;
     for (int i0 = n - 3; i0 >= 0; i0 -= DGTSV_SWEEP_PF) {
         double bvv[DGTSV_SWEEP_PF], duv[DGTSV_SWEEP_PF], dlv[DGTSV_SWEEP_PF], dv[DGTSV_SWEEP_PF];
+        double rv[DGTSV_SWEEP_PF];
 #pragma unroll
         for (int u = 0; u < DGTSV_SWEEP_PF; u++) {
             const int ii = i0 - u > 0 ? i0 - u : 0;
@@ -207,19 +252,48 @@ __host__ __device__ inline void dgtsv_sweeps(int n, const double *F, double *bv,
             duv[u] = du[ii];
             dlv[u] = dl[ii];
             dv[u] = d[ii];
+            rv[u] = rec ? rec[ii] : 0.0;
         }
+        bool ok = rec != nullptr;
+        const double xs = x_next, xs2 = x_next2;
+        if (ok) {
 #pragma unroll
-        for (int u = 0; u < DGTSV_SWEEP_PF; u++) {
-            const int ii = i0 - u;
-            if (ii >= 0) {
-                const double xi = (bvv[u] - duv[u] * x_next - dlv[u] * x_next2) / dv[u];
-                SB(ii) = xi;
-                x_next2 = x_next;
-                x_next = xi;
+            for (int u = 0; u < DGTSV_SWEEP_PF; u++) {
+                const int ii = i0 - u;
+                if (ii >= 0) {
+                    const double a = bvv[u] - duv[u] * x_next - dlv[u] * x_next2;
+                    ok = ok & div_in_range(a) & div_in_range(dv[u]);
+                    const double xi = div_by_reciprocal(a, dv[u], rv[u]);
+                    SB(ii) = xi;
+                    x_next2 = x_next;
+                    x_next = xi;
+                }
             }
         }
+        if (!ok) {
+            x_next = xs;
+            x_next2 = xs2;
+#pragma unroll
+            for (int u = 0; u < DGTSV_SWEEP_PF; u++) {
+                const int ii = i0 - u;
+                if (ii >= 0) {
+                    const double xi = (bvv[u] - duv[u] * x_next - dlv[u] * x_next2) / dv[u];
+                    SB(ii) = xi;
+                    x_next2 = x_next;
+                    x_next = xi;
+                }
+            }
+        }
+        done(i0 - DGTSV_SWEEP_PF + 1 > 0 ? i0 - DGTSV_SWEEP_PF + 1 : 0);
     }
 #undef SB
+}
+
+// Both sweeps with divisions.
+__host__ __device__ inline void dgtsv_sweeps(int n, const double *F, double *bv, long bs)
+{
+    dgtsv_forward(n, F, bv, bs, DgtsvNoHook());
+    dgtsv_back(n, F, nullptr, bv, bs, DgtsvNoHook());
 }
 
 }  // namespace few

@@ -371,6 +371,22 @@ void twin_dgtsv_pair(int n, const double *d, const double *du, const double *dl,
     }
 }
 
+// The back substitution with divisions (x_div) and with the reciprocals of the
+// diagonal (x_rec) on one triangle F = piv | fact | d | du | dl, right-hand side b;
+// q[i] = div_by_reciprocal(b[i], d[i], 1 / d[i]).
+void twin_dgtsv_back_pair(int n, const double *F, const double *b, double *x_div, double *x_rec,
+                          double *q)
+{
+    std::vector<double> rec(n);
+    for (int i = 0; i < n; i++) {
+        rec[i] = 1.0 / F[2 * n + i];
+        x_div[i] = x_rec[i] = b[i];
+        q[i] = div_by_reciprocal(b[i], F[2 * n + i], rec[i]);
+    }
+    dgtsv_back(n, F, nullptr, x_div, 1, DgtsvNoHook());
+    dgtsv_back(n, F, rec.data(), x_rec, 1, DgtsvNoHook());
+}
+
 void twin_sincos_circle(const double *f, double *s, double *c, long n)
 {
     for (long i = 0; i < n; i++) sincos_turns_circle(reduce_turns(f[i]), s[i], c[i]);
