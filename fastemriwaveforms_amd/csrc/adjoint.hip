@@ -340,16 +340,7 @@ __global__ __launch_bounds__(256) void spline_adjoint_lds_kernel(SplineAdjArgs a
         }
     }
     __syncthreads();
-    if (wv == 0) {
-        if (half == 0) dgtsv_forward(L, F, sS + ls, S, DgtsvNoHook());
-        // the reciprocals over the elimination's factors, which are spent
-        double *rec = F + L;
-        const double *d = F + 2L * L;
-        for (int r = lane; r < L; r += 64) rec[r] = 1.0 / d[r];
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (half == 0) dgtsv_back(L, F, rec, sS + ls, S, DgtsvNoHook());
-    }
+    if (wv == 0 && half == 0) dgtsv_sweeps(L, F, sS + ls, S);
     __syncthreads();
     if (ls >= nloc) return;
     {
