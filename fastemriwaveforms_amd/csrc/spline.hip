@@ -522,10 +522,21 @@ __host__ __device__ void spline_one_system(const SplineArgs &a, int gi, int s)
 #define SPLINE_BLOCK 256  // threads of the shared-knot block (4 waves)
 #define SPLINE_SPB 32     // systems per shared-knot block (half a wave)
 
-// Progress counters of a shared-knot block (LDS), one writer each; the readers
-// spin on them, and every writer runs to its end whatever the readers do.
+// Progress counters of a shared-knot block (LDS), one writing wave each; the
+// readers spin on them, and every writer runs to its end whatever the readers do.
+//
+// The store says that every lane of the writing wave is past its LDS stores so
+// far, also where they sit in a branch only some lanes took just before (the
+// repair in dgtsv_back) or in a loop with another trip count per half.  A lane's
+// release orders that lane's own stores only, and an ordinary store may be copied
+// into both arms of such a branch, where the first arm's lanes would publish rows
+// the others still rewrite.  The wave barrier may not be copied: the lanes are
+// together after it, their stores before it ordered by the fence, and all write
+// the same value (from one lane only, the branch costs 2 % of a 120-knot build).
 __device__ __forceinline__ void spline_post(int *c, int v)
 {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     __hip_atomic_store(c, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 __device__ __forceinline__ int spline_peek(int *c)
