@@ -882,17 +882,12 @@ __global__ __launch_bounds__(64) void fd_index_kernel(FdArgs a, CellIndex cells,
     if (lane == 0) ix.cnt[c] = cnt;
 }
 
-// The items of every (cell, segment) (FdSeg's first part) and of every segment
-// (the rest), so that the sum fetches an item with two loads per lane.
-__global__ __launch_bounds__(256) void fd_table_kernel(FdArgs a, CellIndex cells, double *cell_tab,
-                                                       double *seg_tab)
+// The item of (cell c, segment j): its first mode's segment and the combined
+// cubics of its members.
+__device__ inline void fd_form_item(const FdArgs &a, const CellIndex &cells, int c, int j, FdSeg &v)
 {
-    const long at = (long)blockIdx.x * 256 + threadIdx.x;
-    const int c = (int)(at / a.nseg), j = (int)(at - (long)c * a.nseg);
-    if (c >= (cells.start ? *cells.count : a.K)) return;
     const int s0 = cells.start ? cells.start[c] : c, s1 = cells.start ? cells.start[c + 1] : c + 1;
     const long nb = (2L * a.K + 3) * a.L;
-    FdSeg v;
     fd_load_seg(a, cells.start ? cells.member[s0] : c, j, v);
     fcx cp[4], cm[4];
 #pragma unroll
@@ -912,13 +907,26 @@ __global__ __launch_bounds__(256) void fd_table_kernel(FdArgs a, CellIndex cells
         v.tab[4 * p + 3] = cm[p].im;
     }
     v.pad[0] = v.pad[1] = v.pad2[0] = v.pad2[1] = v.pad2[2] = 0.0;
+}
+
+// The items of every segment of the cells [c0, c0 + ncells) (FdSeg's first part)
+// and, with cell 0, of every segment (the rest), so that the sum fetches an item
+// with two loads per lane.
+__global__ __launch_bounds__(256) void fd_table_kernel(FdArgs a, CellIndex cells, int c0, int ncells,
+                                                       double *cell_tab, double *seg_tab)
+{
+    const long at = (long)blockIdx.x * 256 + threadIdx.x;
+    const int i = (int)(at / a.nseg), j = (int)(at - (long)i * a.nseg), c = c0 + i;
+    if (i >= ncells || c >= (cells.start ? *cells.count : a.K)) return;
+    FdSeg v;
+    fd_form_item(a, cells, c, j, v);
     const double *d = reinterpret_cast<const double *>(&v);
 #pragma unroll
-    for (int i = 0; i < FD_CELL_DOUBLES; i++) cell_tab[FD_CELL_DOUBLES * at + i] = d[i];
+    for (int e = 0; e < FD_CELL_DOUBLES; e++) cell_tab[FD_CELL_DOUBLES * at + e] = d[e];
     if (c == 0) {
 #pragma unroll
-        for (int i = 0; i < FD_SEG_DOUBLES; i++)
-            seg_tab[FD_SEG_DOUBLES * j + i] = d[FD_CELL_DOUBLES + i];
+        for (int e = 0; e < FD_SEG_DOUBLES; e++)
+            seg_tab[FD_SEG_DOUBLES * j + e] = d[FD_CELL_DOUBLES + e];
     }
 }
 
@@ -945,12 +953,16 @@ __device__ inline void fd_candidates(const FdOwnIndex &ix, long base, int c, int
     s = l;
 }
 
-template <int BPT>
+// Cells [c0, c0 + ncells).  TABLE: items from fd_table_kernel's tables of these
+// cells; otherwise a wave's first lane forms each (workspaces without tables).
+template <int BPT, bool TABLE>
 __global__ __launch_bounds__(FD_OWN_TILE) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void fd_own_kernel(FdArgs a, CellIndex cells, const double *cell_tab, const double *seg_tab,
-                   FdOwnIndex ix, int n_low, int hb0, int tiles_low)
+void fd_own_kernel(FdArgs a, CellIndex cells, int c0, int ncells, const double *cell_tab,
+                   const double *seg_tab, FdOwnIndex ix, int n_low, int hb0, int tiles_low)
 {
     constexpr int SPAN = 64 * BPT;  // owners per tile
+    const int ncell = min(cells.start ? *cells.count : a.K, c0 + ncells);
+    if (c0 >= ncell) return;  // uniform over the grid: fewer cells than modes
     __shared__ int s_q[2 * FD_OWN_TILE], s_s[2 * FD_OWN_TILE], s_e[2 * FD_OWN_TILE];
     __shared__ int s_scan[FD_OWN_TILE];
     __shared__ FdSeg s_it[FD_OWN_TILE / 64];  // the item each wave evaluates
@@ -985,8 +997,7 @@ void fd_own_kernel(FdArgs a, CellIndex cells, const double *cell_tab, const doub
     const FdSpaConst kc = fd_spa_const();
     const FdRootConst kr = fd_root_const();
     const bool minus_on = a.include_minus_m != 0;
-    const int ncell = cells.start ? *cells.count : a.K;
-    for (int q0 = 0; q0 < ncell; q0 += FD_OWN_TILE) {
+    for (int q0 = c0; q0 < ncell; q0 += FD_OWN_TILE) {
         // candidate segment ranges of cell q0 + tid, compacted in cell order
         const int q = q0 + tid;
         int sa = 0, ea = 0, sb = 0, eb = 0;
@@ -1054,10 +1065,15 @@ void fd_own_kernel(FdArgs a, CellIndex cells, const double *cell_tab, const doub
                 if (!__any(mask != 0)) continue;
                 // the item's values, one copy per wave in LDS
                 __builtin_amdgcn_wave_barrier();
-                double *d = reinterpret_cast<double *>(&it);
-                if (lane < FD_CELL_DOUBLES) d[lane] = cell_tab[FD_CELL_DOUBLES * (base + j) + lane];
-                if (lane < FD_SEG_DOUBLES)
-                    d[FD_CELL_DOUBLES + lane] = seg_tab[FD_SEG_DOUBLES * j + lane];
+                if (TABLE) {
+                    double *d = reinterpret_cast<double *>(&it);
+                    const long at = (long)(qe - c0) * a.nseg + j;
+                    if (lane < FD_CELL_DOUBLES) d[lane] = cell_tab[FD_CELL_DOUBLES * at + lane];
+                    if (lane < FD_SEG_DOUBLES)
+                        d[FD_CELL_DOUBLES + lane] = seg_tab[FD_SEG_DOUBLES * j + lane];
+                } else if (lane == 0) {
+                    fd_form_item(a, cells, qe, j, it);
+                }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
 #pragma nounroll
@@ -1137,23 +1153,58 @@ static size_t fd_scan_ws_bytes(int K, int nseg)
     return sizeof(long) * (size_t)(2 * nitems + 1 + nb + 1);
 }
 
-size_t fd_workspace_bytes(int K, int nseg)
+// What either path takes at least: the scan of the item walk (separate_modes)
+// and the index of the bin-owned sum.
+static size_t fd_base_bytes(int K, int nseg)
 {
     const size_t nitems = (size_t)K * nseg;
-    // the item-walk scan (separate_modes) and the bin-owned index share nothing
     return fd_align256(fd_scan_ws_bytes(K, nseg)) + fd_align256(sizeof(int) * (size_t)K) +
-           3 * fd_align256(sizeof(int) * nitems) + fd_align256(FD_CELL_DOUBLES * sizeof(double) * nitems) +
-           fd_align256(FD_SEG_DOUBLES * sizeof(double) * (size_t)nseg) +
-           cell_index_bytes(K);
+           3 * fd_align256(sizeof(int) * nitems);
+}
+
+// Bin-owned sum: its index, the cells and the tables, from the workspace's start
+// (the item walk's scan is not used there).  The number of cells is known on the
+// device only, so the tables are sized for a slab of cells and the sum runs once
+// per slab the modes could fill; past the last cell a launch ends at once.  64 MB
+// hold 1762 cells of 119 segments, all 671 of the l <= 10, |n| <= 30 set: 3843
+// modes in 0.02 yr take 559 us with the two empty passes and 551 us with tables
+// for a cell per mode (146 MB).
+#define FD_TABLE_BYTES ((size_t)1 << 26)
+
+struct FdOwnLayout {
+    size_t cnt, slo, sj, pmx, cells, seg, tab, total;
+    int slab;  // cells per pass
+};
+
+static FdOwnLayout fd_own_layout(int K, int nseg)
+{
+    const size_t nitems = (size_t)K * nseg;
+    const size_t per_cell = FD_CELL_DOUBLES * sizeof(double) * (size_t)nseg;
+    FdOwnLayout l;
+    l.cnt = 0;
+    l.slo = fd_align256(sizeof(int) * (size_t)K);
+    l.sj = l.slo + fd_align256(sizeof(int) * nitems);
+    l.pmx = l.sj + fd_align256(sizeof(int) * nitems);
+    l.cells = l.pmx + fd_align256(sizeof(int) * nitems);
+    l.seg = l.cells + (K >= CELL_MIN_MODES ? cell_index_bytes(K) : 0);
+    l.tab = l.seg + fd_align256(FD_SEG_DOUBLES * sizeof(double) * (size_t)nseg);
+    l.slab = (int)std::min((size_t)K, std::max(FD_TABLE_BYTES / std::max(per_cell, (size_t)1), (size_t)1));
+    l.total = l.tab + fd_align256(per_cell * (size_t)l.slab);
+    return l;
+}
+
+size_t fd_workspace_bytes(int K, int nseg)
+{
+    return std::max(fd_base_bytes(K, nseg), fd_own_layout(K, nseg).total);
 }
 
 int launch_fd_sum(FdArgs a, void *workspace, size_t workspace_bytes, hipStream_t stream)
 {
     const long nitems = (long)a.K * a.nseg;
     if (nitems <= 0) return FEW_OK;
-    if (workspace_bytes < fd_workspace_bytes(a.K, a.nseg)) {
+    if (workspace_bytes < fd_base_bytes(a.K, a.nseg)) {
         set_error("fd_sum: workspace of %zu bytes, need %zu", workspace_bytes,
-                  fd_workspace_bytes(a.K, a.nseg));
+                  fd_base_bytes(a.K, a.nseg));
         return FEW_ERR_ARG;
     }
     const long nb = (nitems + FD_SCAN_BLOCK - 1) / FD_SCAN_BLOCK;
@@ -1162,43 +1213,49 @@ int launch_fd_sum(FdArgs a, void *workspace, size_t workspace_bytes, hipStream_t
         return FEW_ERR_LIMIT;
     }
     if (!a.separate_modes) {
-        // bin-owned: every bin written once, contributions in a fixed order
-        char *w = static_cast<char *>(workspace) + fd_align256(fd_scan_ws_bytes(a.K, a.nseg));
+        // bin-owned: every bin written once per slab, contributions in a fixed order
+        const FdOwnLayout l = fd_own_layout(a.K, a.nseg);
+        char *w = static_cast<char *>(workspace);
         FdOwnIndex ix;
-        ix.cnt = reinterpret_cast<int *>(w);
-        w += fd_align256(sizeof(int) * (size_t)a.K);
-        ix.slo = reinterpret_cast<int *>(w);
-        w += fd_align256(sizeof(int) * (size_t)nitems);
-        ix.sj = reinterpret_cast<int *>(w);
-        w += fd_align256(sizeof(int) * (size_t)nitems);
-        ix.pmx = reinterpret_cast<int *>(w);
-        w += fd_align256(sizeof(int) * (size_t)nitems);
-        double *cell_tab = reinterpret_cast<double *>(w);
-        w += fd_align256(FD_CELL_DOUBLES * sizeof(double) * (size_t)nitems);
-        double *seg_tab = reinterpret_cast<double *>(w);
-        w += fd_align256(FD_SEG_DOUBLES * sizeof(double) * (size_t)a.nseg);
+        ix.cnt = reinterpret_cast<int *>(w + l.cnt);
+        ix.slo = reinterpret_cast<int *>(w + l.slo);
+        ix.sj = reinterpret_cast<int *>(w + l.sj);
+        ix.pmx = reinterpret_cast<int *>(w + l.pmx);
+        double *seg_tab = reinterpret_cast<double *>(w + l.seg);
+        double *cell_tab = reinterpret_cast<double *>(w + l.tab);
         CellIndex cells;
-        if (a.K >= CELL_MIN_MODES) {
-            int rc = launch_cell_index(a.m, a.k, a.n, a.K, a.seg_start, a.seg_end, a.nseg, w, cells,
-                                       stream);
+        if (a.K >= CELL_MIN_MODES && workspace_bytes >= l.seg) {
+            int rc = launch_cell_index(a.m, a.k, a.n, a.K, a.seg_start, a.seg_end, a.nseg,
+                                       w + l.cells, cells, stream);
             if (rc) return rc;
         }
         hipLaunchKernelGGL(fd_index_kernel, dim3(a.K), dim3(64), 0, stream, a, cells, ix);
         FEW_HIP(hipGetLastError());
-        hipLaunchKernelGGL(fd_table_kernel, dim3((unsigned)((nitems + 255) / 256)), dim3(256), 0,
-                           stream, a, cells, cell_tab, seg_tab);
-        FEW_HIP(hipGetLastError());
+        // a workspace between the least and the one asked for holds no tables
+        const bool tables = workspace_bytes >= l.total;
+        const int slab = tables ? l.slab : a.K;
         int n_low, hb0, tiles_low, tiles;
-        const int bpt = std::max(a.zero_index + 1, a.data_length - a.zero_index) < FD_OWN_LONG ? 1 : 2;
+        const int bpt = tables && std::max(a.zero_index + 1, a.data_length - a.zero_index) >= FD_OWN_LONG
+                            ? 2 : 1;
         fd_owner_split(a.zero_index, a.data_length, bpt, n_low, hb0, tiles_low, tiles);
-        if (tiles > 0) {
-            const dim3 grid(tiles), block(FD_OWN_TILE);
+        const dim3 grid(tiles), block(FD_OWN_TILE);
+        for (int c0 = 0; c0 < a.K && tiles > 0; c0 += slab) {
+            if (!tables) {
+                hipLaunchKernelGGL((fd_own_kernel<1, false>), grid, block, 0, stream, a, cells, c0,
+                                   slab, cell_tab, seg_tab, ix, n_low, hb0, tiles_low);
+                FEW_HIP(hipGetLastError());
+                break;
+            }
+            const long items = (long)std::min(slab, a.K - c0) * a.nseg;
+            hipLaunchKernelGGL(fd_table_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0,
+                               stream, a, cells, c0, slab, cell_tab, seg_tab);
+            FEW_HIP(hipGetLastError());
             if (bpt == 1)
-                hipLaunchKernelGGL(fd_own_kernel<1>, grid, block, 0, stream, a, cells, cell_tab,
-                                   seg_tab, ix, n_low, hb0, tiles_low);
+                hipLaunchKernelGGL((fd_own_kernel<1, true>), grid, block, 0, stream, a, cells, c0,
+                                   slab, cell_tab, seg_tab, ix, n_low, hb0, tiles_low);
             else
-                hipLaunchKernelGGL(fd_own_kernel<2>, grid, block, 0, stream, a, cells, cell_tab,
-                                   seg_tab, ix, n_low, hb0, tiles_low);
+                hipLaunchKernelGGL((fd_own_kernel<2, true>), grid, block, 0, stream, a, cells, c0,
+                                   slab, cell_tab, seg_tab, ix, n_low, hb0, tiles_low);
             FEW_HIP(hipGetLastError());
         }
         return FEW_OK;

@@ -22,7 +22,9 @@ struct FdArgs {
     int include_minus_m, separate_modes;
 };
 
-// Workspace: the per-(mode, segment) bin counts and their prefix.
+// Workspace: the bin counts and their prefix (separate_modes), or the sorted segments
+// of every cell and the tables of at most 64 MB of cells.  The sum also runs in the
+// first's 28 B per (mode, segment) (fd_base_bytes), then without the tables.
 size_t fd_workspace_bytes(int K, int nseg);
 int launch_fd_sum(FdArgs a, void *workspace, size_t workspace_bytes, hipStream_t stream);
 

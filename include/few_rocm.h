@@ -314,8 +314,11 @@ int few_direct_mode_sum_async(const void *teuk, const void *ylms, const double *
 
 /* ---- frequency-domain interpolated sum --------------------------------- */
 
-/* Bytes of workspace few_get_waveform_generic_fd_async needs (the per-(mode,
- * segment) bin counts and their prefix): written to *bytes. */
+/* Bytes of workspace for few_get_waveform_generic_fd_async, written to *bytes:
+ * 28 B per (mode, segment) for the per-segment index, plus at most 64 MB of
+ * per-(cell, segment) tables.  The call itself takes any workspace from 28 B per
+ * (mode, segment) on (each of its arrays rounded up to 256 B); with less than
+ * the size given here the sum forms the tables' values as it goes. */
 int few_fd_workspace_bytes(int num_teuk_modes, int num_segments, size_t *bytes);
 
 /* Replaces get_waveform_generic_fd (src/few/cutils/interpolate.hh:33-38,
