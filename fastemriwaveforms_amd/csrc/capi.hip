@@ -399,7 +399,7 @@ static int run_waveform(double2 *wave, const double *interp, const double *pt, c
         set_error("get_waveform: precision %d is not supported", precision);
         return FEW_ERR_UNSUPPORTED;
     }
-    const int tile = direct_tile(out_len);
+    const int tile = direct_tile(out_len, K);
     const PrepKey key{ws, plan, precision, tile, L, out_len};
     if (int rc = prep_stage(stage & 1, stage & 2, key, "get_waveform")) return rc;
     if (stage & 1) {

@@ -112,102 +112,126 @@ struct DirectLds {
     double mkn[3][CELL_CH];
 };
 
-// The cell loop of a tile: this wave's partial sums (re, im) of its samples.
+// Stages cells [c0, c0 + cnt) of interval j (all four waves; the caller syncs).
+__device__ __forceinline__ void direct_stage(const DirectArgs &a, int j, int c0, int cnt, DirectLds &sh)
+{
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // power staged
+    const int own = threadIdx.x & 63;                                   // cell staged
+    const int K = a.K;
+    const double *ip = a.interp + (long)part * ((long)a.L * 2 * K) + (long)j * 2 * K;
+    if (own < cnt) {
+        int s0 = c0 + own, s1 = s0 + 1;
+        if (a.cells.start) {
+            s0 = a.cells.start[c0 + own];
+            s1 = a.cells.start[c0 + own + 1];
+        }
+        const int lead = a.cells.start ? a.cells.member[s0] : s0;
+        const int m = a.m[lead];
+        double v[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int s = s0; s < s1; s++) {
+            const int mode = a.cells.start ? a.cells.member[s] : s;
+            const double2 yp = a.ylm[mode], ym = a.ylm[K + mode];
+            cell_coef_add(ip[mode], ip[K + mode], yp.x, yp.y, ym.x, ym.y, m != 0, v);
+        }
+        sh.c[part][own] = make_double4(v[0], v[1], v[2], v[3]);
+        if (part == 0)
+            sh.mkn[0][own] = (double)m;
+        else if (part == 1)
+            sh.mkn[1][own] = (double)a.k[lead];
+        else if (part == 2)
+            sh.mkn[2][own] = (double)a.n[lead];
+    }
+}
+
+// Adds the staged cells first, first + STEP, ... below cnt to the samples' sums.
 // Returns whether every phase was within sincos_half_turns' range (always, if BIG).
+template <int SPT, bool BIG, int STEP>
+__device__ __forceinline__ bool direct_add(const DirectLds &sh, int first, int cnt,
+                                           const double (&x)[SPT], const double (&Pp)[SPT],
+                                           const double (&Pt)[SPT], const double (&Pr)[SPT],
+                                           double (&re)[SPT], double (&im)[SPT])
+{
+    bool ok = true;
+    for (int jj = first; jj < cnt; jj += STEP) {
+        double c[4][4];
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const double4 t = sh.c[p][jj];
+            c[p][0] = t.x;
+            c[p][1] = t.y;
+            c[p][2] = t.z;
+            c[p][3] = t.w;
+        }
+        const double m = sh.mkn[0][jj], k = sh.mkn[1][jj], n = sh.mkn[2][jj];
+#pragma unroll
+        for (int u = 0; u < SPT; u++) {
+            const bool in = cell_term_fp64<BIG>(c, m, k, n, x[u], Pp[u], Pt[u], Pr[u], re[u], im[u]);
+            ok = ok && in;
+        }
+    }
+    return ok;
+}
+
+// The cell loop of a tile: this wave's partial sums (re, im) of its samples, over
+// every fourth cell.
 template <int SPT, bool BIG>
 __device__ __forceinline__ bool direct_cells(const DirectArgs &a, int j, DirectLds &sh,
                                              const double (&x)[SPT], const double (&Pp)[SPT],
                                              const double (&Pt)[SPT], const double (&Pr)[SPT],
                                              double (&re)[SPT], double (&im)[SPT])
 {
-    const int tid = threadIdx.x;
-    const int part = __builtin_amdgcn_readfirstlane(tid >> 6);  // power staged, cells summed
-    const int own = tid & 63;                                   // cell staged
-    const int K = a.K;
-    const long nb = (long)a.L * 2 * K;
-    const double *ip = a.interp + (long)part * nb + (long)j * 2 * K;
-    const int ncell = a.cells.start ? *a.cells.count : K;
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ncell = a.cells.start ? *a.cells.count : a.K;
     bool ok = true;
 #pragma unroll
     for (int u = 0; u < SPT; u++) re[u] = im[u] = 0.0;
     for (int c0 = 0; c0 < ncell; c0 += CELL_CH) {
         const int cnt = min(CELL_CH, ncell - c0);
         __syncthreads();
-        if (own < cnt) {
-            int s0 = c0 + own, s1 = s0 + 1;
-            if (a.cells.start) {
-                s0 = a.cells.start[c0 + own];
-                s1 = a.cells.start[c0 + own + 1];
-            }
-            const int lead = a.cells.start ? a.cells.member[s0] : s0;
-            const int m = a.m[lead];
-            double v[4] = {0.0, 0.0, 0.0, 0.0};
-            for (int s = s0; s < s1; s++) {
-                const int mode = a.cells.start ? a.cells.member[s] : s;
-                const double2 yp = a.ylm[mode], ym = a.ylm[K + mode];
-                cell_coef_add(ip[mode], ip[K + mode], yp.x, yp.y, ym.x, ym.y, m != 0, v);
-            }
-            sh.c[part][own] = make_double4(v[0], v[1], v[2], v[3]);
-            if (part == 0)
-                sh.mkn[0][own] = (double)m;
-            else if (part == 1)
-                sh.mkn[1][own] = (double)a.k[lead];
-            else if (part == 2)
-                sh.mkn[2][own] = (double)a.n[lead];
-        }
+        direct_stage(a, j, c0, cnt, sh);
         __syncthreads();
-        for (int jj = part; jj < cnt; jj += 4) {
-            double c[4][4];
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-                const double4 t = sh.c[p][jj];
-                c[p][0] = t.x;
-                c[p][1] = t.y;
-                c[p][2] = t.z;
-                c[p][3] = t.w;
-            }
-            const double m = sh.mkn[0][jj], k = sh.mkn[1][jj], n = sh.mkn[2][jj];
-#pragma unroll
-            for (int u = 0; u < SPT; u++) {
-                const bool in = cell_term_fp64<BIG>(c, m, k, n, x[u], Pp[u], Pt[u], Pr[u], re[u],
-                                                    im[u]);
-                ok = ok && in;
-            }
-        }
+        const bool in = direct_add<SPT, BIG, 4>(sh, part, cnt, x, Pp, Pt, Pr, re, im);
+        ok = ok && in;
     }
     return ok;
 }
 
-template <int SPT>
-__device__ __forceinline__ void direct_fp64_tile(const DirectArgs &a, int j, int q)
+// Sample state of this lane's samples base + u STEP (those past the interval
+// repeat its last one; their sums are dropped).
+template <int SPT, int STEP>
+__device__ __forceinline__ void direct_samples(const DirectArgs &a, int j, const Segment &sg, int base,
+                                               double (&x)[SPT], double (&Pp)[SPT],
+                                               double (&Pt)[SPT], double (&Pr)[SPT])
 {
-    __shared__ DirectLds sh;
+    const long np = (long)a.nseg * 3;
+    double rp[8], rt[8], rr[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        rp[c] = a.pcoef[c * np + (long)j * 3 + 0];
+        rt[c] = a.pcoef[c * np + (long)j * 3 + 1];
+        rr[c] = a.pcoef[c * np + (long)j * 3 + 2];
+    }
+#pragma unroll
+    for (int u = 0; u < SPT; u++) {
+        SampleState st;
+        sample_state(a.dt, min(base + u * STEP, sg.end - 1), sg.h_t, sg.pt, sg.pw, rp, rt, rr, st);
+        x[u] = st.x;
+        Pp[u] = st.Pp;
+        Pt[u] = st.Pt;
+        Pr[u] = st.Pr;
+    }
+}
+
+template <int SPT>
+__device__ __forceinline__ void direct_fp64_tile(const DirectArgs &a, int j, int q, DirectLds &sh)
+{
     __shared__ double2 s_sum[3][64 * SPT];
     const int tid = threadIdx.x, lane = tid & 63;
     const int part = __builtin_amdgcn_readfirstlane(tid >> 6);
     const Segment sg = a.segs[j];
     const int base = sg.start + q * (64 * SPT) + lane;
     double x[SPT], Pp[SPT], Pt[SPT], Pr[SPT], re[SPT], im[SPT];
-    {
-        const long np = (long)a.nseg * 3;
-        double rp[8], rt[8], rr[8];
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            rp[c] = a.pcoef[c * np + (long)j * 3 + 0];
-            rt[c] = a.pcoef[c * np + (long)j * 3 + 1];
-            rr[c] = a.pcoef[c * np + (long)j * 3 + 2];
-        }
-#pragma unroll
-        for (int u = 0; u < SPT; u++) {
-            SampleState st;
-            // samples past the interval repeat its last one (their sums are dropped)
-            sample_state(a.dt, min(base + u * 64, sg.end - 1), sg.h_t, sg.pt, sg.pw, rp, rt, rr, st);
-            x[u] = st.x;
-            Pp[u] = st.Pp;
-            Pt[u] = st.Pt;
-            Pr[u] = st.Pr;
-        }
-    }
+    direct_samples<SPT, 64>(a, j, sg, base, x, Pp, Pt, Pr);
     const bool ok = direct_cells<SPT, false>(a, j, sh, x, Pp, Pt, Pr, re, im);
     // phases beyond 1e8 rad (or NaN): the tile again with the library's sincos
     if (__syncthreads_or(!ok)) direct_cells<SPT, true>(a, j, sh, x, Pp, Pt, Pr, re, im);
@@ -234,7 +258,76 @@ __device__ __forceinline__ void direct_fp64_tile(const DirectArgs &a, int j, int
     }
 }
 
-// Overwriting sum: samples past the last interval's are zero.
+// All staged cells for the lane's own samples, summed as the four waves of
+// direct_fp64_tile sum them: every fourth cell, then the four sums in pairs.
+template <int SPT, bool BIG>
+__device__ __forceinline__ bool direct_few_cells(const DirectLds &sh, int cnt, const double (&x)[SPT],
+                                                 const double (&Pp)[SPT], const double (&Pt)[SPT],
+                                                 const double (&Pr)[SPT], double (&re)[SPT],
+                                                 double (&im)[SPT])
+{
+    bool ok = true;
+    double r[SPT], i[SPT], pr[SPT], pi[SPT];  // this part's sum, the even part before it
+#pragma unroll
+    for (int u = 0; u < SPT; u++) re[u] = im[u] = 0.0;
+#pragma nounroll
+    for (int part = 0; part < 4; part++) {
+#pragma unroll
+        for (int u = 0; u < SPT; u++) r[u] = i[u] = 0.0;
+        const bool in = direct_add<SPT, BIG, 4>(sh, part, cnt, x, Pp, Pt, Pr, r, i);
+        ok = ok && in;
+#pragma unroll
+        for (int u = 0; u < SPT; u++) {
+            re[u] = part & 1 ? re[u] + (pr[u] + r[u]) : re[u];
+            im[u] = part & 1 ? im[u] + (pi[u] + i[u]) : im[u];
+            pr[u] = r[u];
+            pi[u] = i[u];
+        }
+    }
+    return ok;
+}
+
+// One tile (256 SPT samples) of a set of few modes: every lane has samples of its
+// own and sums all cells, what the output holds being read ahead of them.  Four
+// waves on the same samples would form each sample's state four times, which is
+// most of the work here: one mode, 3.2 million samples added to: 34 us (66 us with
+// direct_fp64_tile), 12 modes 82 us (102 us).  The same bits either way.
+//
+// What bounds it: with one mode the latency of a workgroup's chain (search, loads,
+// staging, one sincos), 3.0 TB/s of the output read and written; from about ten
+// modes FP64 VALU issue.
+template <int SPT>
+__device__ __forceinline__ void direct_few_tile(const DirectArgs &a, int j, int q, DirectLds &sh)
+{
+    static_assert(DIRECT_FEW <= CELL_CH && DIRECT_FEW < CELL_MIN_MODES,
+                  "one staging holds every cell, a cell per mode");
+    const Segment sg = a.segs[j];
+    const int base = sg.start + q * (256 * SPT) + threadIdx.x;
+    double x[SPT], Pp[SPT], Pt[SPT], Pr[SPT], re[SPT], im[SPT];
+    double2 o[SPT];
+#pragma unroll
+    for (int u = 0; u < SPT; u++) {
+        const int idx = base + u * 256;
+        o[u] = !a.overwrite && idx < sg.end ? a.wave[idx] : make_double2(0.0, 0.0);
+    }
+    direct_stage(a, j, 0, a.K, sh);
+    direct_samples<SPT, 256>(a, j, sg, base, x, Pp, Pt, Pr);
+    __syncthreads();
+    if (!__all(direct_few_cells<SPT, false>(sh, a.K, x, Pp, Pt, Pr, re, im)))
+        direct_few_cells<SPT, true>(sh, a.K, x, Pp, Pt, Pr, re, im);
+#pragma unroll
+    for (int u = 0; u < SPT; u++) {
+        const int idx = base + u * 256;
+        if (idx >= sg.end) continue;
+        a.wave[idx] = a.overwrite ? make_double2(re[u], im[u])
+                                  : make_double2(re[u] + o[u].x, im[u] + o[u].y);
+    }
+}
+
+// Overwriting sum: samples past the last interval's are zero.  Called after the
+// tile: with a store to the output ahead of it, the compiler would take the tile's
+// uniform values (interval, phase coefficients) through vector loads, lane by lane
+// (one mode, 3.2 million samples: 43 us instead of 32).
 __device__ __forceinline__ void direct_zero_tail(const DirectArgs &a, long block, long blocks)
 {
     const long end = a.nseg > 0 ? a.segs[a.nseg - 1].end : 0;
@@ -242,16 +335,32 @@ __device__ __forceinline__ void direct_zero_tail(const DirectArgs &a, long block
         a.wave[i] = make_double2(0.0, 0.0);
 }
 
-// Four waves per SIMD (at most 128 registers)
+// Four waves per SIMD: 128 registers, of which the four-sample form spills 51 (208 B
+// of scratch), most of them around the repetition with the library sincos.
 template <int SPT>
 __global__ __launch_bounds__(256, 4) void direct_fp64_kernel(DirectArgs a)
 {
+    __shared__ DirectLds sh;
     const int b = blockIdx.x;
-    if (a.overwrite) direct_zero_tail(a, b, gridDim.x);
     const int total = a.prefix[a.nseg];
-    if (b >= total) return;
-    const int j = find_segment(a.prefix, a.nseg, b);
-    direct_fp64_tile<SPT>(a, j, b - a.prefix[j]);
+    if (b < total) {
+        const int j = find_segment(a.prefix, a.nseg, b);
+        direct_fp64_tile<SPT>(a, j, b - a.prefix[j], sh);
+    }
+    if (a.overwrite) direct_zero_tail(a, b, gridDim.x);
+}
+
+template <int SPT>
+__global__ __launch_bounds__(256, 4) void direct_few_kernel(DirectArgs a)
+{
+    __shared__ DirectLds sh;
+    const int b = blockIdx.x;
+    const int total = a.prefix[a.nseg];
+    if (b < total) {
+        const int j = find_segment(a.prefix, a.nseg, b);
+        direct_few_tile<SPT>(a, j, b - a.prefix[j], sh);
+    }
+    if (a.overwrite) direct_zero_tail(a, b, gridDim.x);
 }
 
 // ------------------------------------------------------------------ batch
@@ -340,7 +449,9 @@ __global__ __launch_bounds__(256, 4) void batch_direct_fp64_kernel(BatchDev B, B
     }
     a.out_len = d.N;
     a.overwrite = 0;
-    direct_fp64_tile<SPT>(a, j, lt - pref[j]);
+    __shared__ DirectLds sh;
+    if (d.K <= DIRECT_FEW) direct_few_tile<SPT / 4>(a, j, lt - pref[j], sh);
+    else direct_fp64_tile<SPT>(a, j, lt - pref[j], sh);
 }
 
 int launch_batch_direct_fp64(const BatchDev &B, const BatchRunDev &r, const BatchPtrs &p,
@@ -364,11 +475,18 @@ int launch_plan(const PlanArgs &p, hipStream_t stream)
     return FEW_OK;
 }
 
-// Below 2^17 samples the four-sample tiles are too few to fill the chip: 63,116
-// samples of the full set take 128 us with one sample per lane and 183 us with
-// four, 315,582 samples of 500 modes 193 us with four and 217 us with one.
-int direct_tile(long out_len)
+// A lane per sample where a set is small and there are samples for the lanes, 4096
+// of them per mode.  Added to an output of 94,675 samples 1 / 8 / 12 / 20 modes take
+// 8.1 / 10.0 / 10.9 / 13.0 us (11.1 / 12.1 / 12.7 / 13.9 with four waves on the same
+// samples), 9468 samples 7.9 / 9.5 / 10.5 / 12.6 us (7.7 / 8.0 / 8.0 / 8.6).
+bool direct_few(long out_len, int K) { return K <= DIRECT_FEW && out_len >= 4096L * K; }
+
+// Otherwise, below 2^17 samples the four-sample tiles are too few to fill the chip:
+// 63,116 samples of the full set take 128 us with one sample per lane and 183 us
+// with four, 315,582 samples of 500 modes 193 us with four and 217 us with one.
+int direct_tile(long out_len, int K)
 {
+    if (direct_few(out_len, K)) return DIRECT_FEW_TILE;
     return out_len < (1L << 17) ? 64 : DIRECT_TILE;
 }
 
@@ -376,7 +494,9 @@ int launch_direct_fp64(const DirectArgs &a, int tile, int max_blocks, hipStream_
 {
     if (max_blocks <= 0) return FEW_OK;
     const dim3 grid(max_blocks);
-    if (tile == DIRECT_TILE)
+    if (tile == DIRECT_FEW_TILE)
+        hipLaunchKernelGGL(direct_few_kernel<DIRECT_FEW_TILE / 256>, grid, dim3(256), 0, stream, a);
+    else if (tile == DIRECT_TILE)
         hipLaunchKernelGGL(direct_fp64_kernel<DIRECT_SPT>, grid, dim3(256), 0, stream, a);
     else
         hipLaunchKernelGGL(direct_fp64_kernel<1>, grid, dim3(256), 0, stream, a);

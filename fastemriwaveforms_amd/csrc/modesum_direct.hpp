@@ -199,8 +199,14 @@ __host__ __device__ inline bool cell_term_fp64(const double (&c)[4][4], double m
 int launch_plan(const PlanArgs &p, hipStream_t stream);
 constexpr int DIRECT_SPT = 4;                  // output samples per lane of a tile
 constexpr int DIRECT_TILE = 64 * DIRECT_SPT;
-// Samples per tile of the FP64 direct sum for an output of out_len samples.
-int direct_tile(long out_len);
+// Sets of at most DIRECT_FEW modes: a lane per sample, in tiles of DIRECT_FEW_TILE
+// samples (a batch keeps DIRECT_TILE).
+constexpr int DIRECT_FEW = 16;
+constexpr int DIRECT_FEW_TILE = 512;
+// Whether the FP64 direct sum of K modes and out_len samples runs that way.
+bool direct_few(long out_len, int K);
+// Samples per tile of the FP64 direct sum of K modes for an output of out_len samples.
+int direct_tile(long out_len, int K);
 int launch_direct_fp64(const DirectArgs &a, int tile, int max_blocks, hipStream_t stream);
 
 }  // namespace few
