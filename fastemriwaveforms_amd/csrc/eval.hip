@@ -84,7 +84,6 @@ __global__ __launch_bounds__(256) void spline_eval_kernel(SplineEvalArgs a)
 #define SE_ARRAYS 64   // arrays of a shared-point tile (lanes of the evaluation)
 #define SE_POINTS 64   // points of a tile (lanes of the search and of the stores)
 #define SE_UNROLL 4    // points in flight per wave (2 and 8 measure the same)
-#define SE_MIN_VALUES (1L << 19)
 
 // Arrays on one set of knots and points, their coefficients array-contiguous
 // (what CubicSplineInterpolant holds): a workgroup takes 64 arrays x 64
@@ -95,10 +94,14 @@ __global__ __launch_bounds__(256) void spline_eval_kernel(SplineEvalArgs a)
 //
 // What bounds it: the writes.  7686 arrays x 1000 points, 120 knots: 30 us,
 // 61 MB written and 30 MB read (105 us with one lane per (array, point), whose
-// four reads fall on 64 different lines per wave).  Tiles of the same arrays run on the same XCD (workgroup i
-// runs on XCD i % 8), whose L2 then holds their coefficients.
+// four reads fall on 64 different lines per wave; 67 us if the points ascend).
+// Workgroup i runs on XCD i % 8, whose L2 holds the coefficients of the groups it
+// works on: every eighth group goes to an XCD, its tiles one after another.  Fewer
+// than 32 groups would leave XCDs with less or no work (64 arrays x 16384 points:
+// 28 us); each XCD then takes an equal run of the tiles instead (9.4 us; for 7686
+// arrays x 256 points such runs cost 5 %, the XCDs being far apart in memory).
 __global__ __launch_bounds__(256) void spline_eval_shared_kernel(SplineEvalArgs a, int chunks,
-                                                                 int groups)
+                                                                 int groups, int per)
 {
     __shared__ double s_v[SE_ARRAYS][SE_POINTS + 1];
     __shared__ double s_x[SE_POINTS];
@@ -106,9 +109,12 @@ __global__ __launch_bounds__(256) void spline_eval_shared_kernel(SplineEvalArgs 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3;
-    const int grp = xcd + 8 * (slot / chunks);
+    const int tile = per ? xcd * per + slot : slot;
+    int grp = tile / chunks;
+    const int q0 = (tile - grp * chunks) * SE_POINTS;
+    if (!per) grp = xcd + 8 * grp;
     if (grp >= groups) return;
-    const int q0 = (slot % chunks) * SE_POINTS, s0 = grp * SE_ARRAYS;
+    const int s0 = grp * SE_ARRAYS;
     const int nq = min(SE_POINTS, a.npts - q0), ns = min(SE_ARRAYS, a.ninterps - s0);
     const int L = a.length;
     if (wv == 0) {
@@ -145,21 +151,36 @@ __global__ __launch_bounds__(256) void spline_eval_shared_kernel(SplineEvalArgs 
     for (int r = wv; r < ns; r += 4) a.out[(long)(s0 + r) * a.npts + q0 + lane] = s_v[r][lane];
 }
 
+// Tiles where they are faster whatever the order of the points (a lane per value
+// reads fewer lines where neighbouring points share an interval).  A tile's search,
+// loads and stores follow each other, so a call in tiles takes 8.8 us or more:
+//                              tiles     lane per value, points ascending / random
+//   512 arrays x 1024 points   8.8       6.6 / 10.1
+//   64 x 16384, 512 x 2048     9.4       10.4, 10.6 / 17.0, 16.9
+//   448 x 2048, 800 x 1024     9.5, 9.1  9.4, 9.2 / 15.0, 14.2
+// and with few points per array the lanes of a wave share less:
+//   1600 x 512, 2048 x 256     9.2, 8.8  9.5, 14.5
+//   1100 x 512                 8.9       7.5
+static bool spline_eval_tiled(const SplineEvalArgs &a, long n)
+{
+    if (a.t_sys != 0 || a.tn_sys != 0 || a.c_sys != 1) return false;
+    if (a.ninterps < SE_ARRAYS || a.npts < SE_POINTS) return false;
+    return n >= 7L << 17 || (a.ninterps >= 1536 && n >= 1L << 19);
+}
+
 int launch_spline_eval(const SplineEvalArgs &a, hipStream_t stream)
 {
     const long n = (long)a.ninterps * a.npts;
     if (n <= 0) return FEW_OK;
-    // Whole tiles in both directions, and enough of them: at 1000 points, 800
-    // arrays take 10.0 us in tiles and 15.0 us with a lane per value, 200 arrays
-    // 9.1 and 5.2 (a tile's search, loads and stores follow each other).
-    if (a.t_sys == 0 && a.tn_sys == 0 && a.c_sys == 1 && a.ninterps >= SE_ARRAYS &&
-        a.npts >= SE_POINTS && n >= SE_MIN_VALUES) {
+    if (spline_eval_tiled(a, n)) {
         const int groups = (a.ninterps + SE_ARRAYS - 1) / SE_ARRAYS;
         const int chunks = (int)(((long)a.npts + SE_POINTS - 1) / SE_POINTS);
-        const long blocks = 8L * ((groups + 7) / 8) * chunks;
+        // 0: every eighth group to an XCD
+        const long per = groups < 32 ? ((long)groups * chunks + 7) / 8 : 0;
+        const long blocks = 8 * (per ? per : (long)((groups + 7) / 8) * chunks);
         if (blocks <= 0x7fffffffL) {
             hipLaunchKernelGGL(spline_eval_shared_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                               stream, a, chunks, groups);
+                               stream, a, chunks, groups, (int)per);
             FEW_HIP(hipGetLastError());
             return FEW_OK;
         }
