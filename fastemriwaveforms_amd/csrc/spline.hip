@@ -34,6 +34,10 @@ namespace few {
 // 80 us (134 / 175 us with a lane per system and its scratch in HBM), 30000 of
 // 290 knots 397 us (534).
 #define SPLINE_SHARED_MAX_L 290
+// Knots from which the chains of a block follow each other (below).  With fewer the
+// counters cost more than the overlap gives: 7686 systems of 8 / 10 / 12 knots 8.5 /
+// 8.7 / 9.0 us following, 7.9 / 8.3 / 9.8 one after the other.
+#define SPLINE_FOLLOW 11
 #define SPLINE_TILE_BATCH 24     // knot-value loads in flight per lane while staging a tile
 
 struct SplineArgs {
@@ -561,8 +565,10 @@ __device__ __forceinline__ int spline_peek(int *c)
 //               reciprocals of the diagonal (dgtsv_back);
 //   waves 1-3:  the coefficients of the intervals and their stores, behind the
 //               back substitution.
+// Below SPLINE_FOLLOW knots the same steps go one after the other, with divisions and
+// the coefficients on all four waves.
 // What bounds it: the latency of those chains, one dependent FP64 operation after
-// another.  7686 systems of 120 knots: 50 us; 30000 of 290 knots: 397 us (57
+// another.  7686 systems of 120 knots: 45 us; 30000 of 290 knots: 397 us (57
 // and 485 us with the chains, 18 us for the elimination and 21 us for the sweeps,
 // and the coefficients one after the other, and a division per step of the back
 // substitution).
@@ -577,6 +583,8 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
     double *sx = lds, *F = sx + n, *sy = F + 5 * n, *sb = sy + (long)n * S;
     // rows eliminated, waves whose right-hand sides are in place, lowest solved row
     __shared__ int s_info, s_elim, s_rhs[2], s_solved;
+    // short chains go one after the other, with divisions and barriers between them
+    const bool follow = n >= SPLINE_FOLLOW;
     const int s0 = blk * S;
     const int nloc = min(S, G.nsys - s0);
     for (int i = tid; i < n; i += SPLINE_BLOCK) sx[i] = G.t[(long)i * G.t_knot];
@@ -600,9 +608,11 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
         const int info = dgtsv_factor_ahead<8>(n, d, du, dl, piv, fact,
-                                               [&](int i) { spline_post(&s_elim, i); });
+                                               [&](int i) {
+                                                   if (follow) spline_post(&s_elim, i);
+                                               });
         if (lane == 0) s_info = info;
-        spline_post(&s_elim, n);
+        if (follow) spline_post(&s_elim, n);
     } else {
         const int c = (n + 2) / 3;
         const int r0 = wv * c, r1 = min(n, r0 + c);
@@ -610,6 +620,8 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
             // knots [k0, k1] hold every value rows r0..r1-1 read; the two
             // halves stage alternate knots
             const int k0 = max(0, min(r0 - 1, n - 3)), k1 = min(n - 1, max(r1, 2));
+            // (lanes past the last system repeat it: zeros would send every group of the
+            // back substitution through its repair)
             const double *ys = G.y + (long)(s0 + min(ls, nloc - 1)) * G.y_sys;
             for (int kb = k0 + half; kb <= k1; kb += 2 * SPLINE_TILE_BATCH) {
                 double v[SPLINE_TILE_BATCH];
@@ -618,7 +630,7 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
                     v[u] = ys[(long)min(kb + 2 * u, k1) * G.y_knot];
 #pragma unroll
                 for (int u = 0; u < SPLINE_TILE_BATCH; u++)
-                    if (kb + 2 * u <= k1) sy[(long)(kb + 2 * u) * S + ls] = ls < nloc ? v[u] : 0.0;
+                    if (kb + 2 * u <= k1) sy[(long)(kb + 2 * u) * S + ls] = v[u];
             }
             // the other half's knots, written by this wave's earlier LDS stores
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -634,17 +646,20 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
             }
         }
     }
-    if (wv == 1 || wv == 2) spline_post(&s_rhs[wv - 1], 1);
+    if (!follow) __syncthreads();
+    else if (wv == 1 || wv == 2) spline_post(&s_rhs[wv - 1], 1);
     if (wv == 0) {
-        while (!spline_peek(&s_rhs[0]) || !spline_peek(&s_rhs[1])) __builtin_amdgcn_s_sleep(1);
+        if (follow)
+            while (!spline_peek(&s_rhs[0]) || !spline_peek(&s_rhs[1])) __builtin_amdgcn_s_sleep(1);
         // after an early return of the elimination this sweeps over rows that
         // mean nothing; the systems are then done one by one below
         if (half == 0)
             dgtsv_forward(n, F, sb + ls, S, [&](int i) {
-                while (spline_peek(&s_elim) < i) __builtin_amdgcn_s_sleep(1);
+                if (follow)
+                    while (spline_peek(&s_elim) < i) __builtin_amdgcn_s_sleep(1);
             });
     }
-    __syncthreads();
+    if (follow) __syncthreads();
     if (s_info != 0) {  // singular: dgtsv's early return, handled system by system
         if (wv == 0 && half == 0) spline_one_system(a, gi, s0 + ls);
         return;
@@ -653,28 +668,37 @@ __device__ void spline_block_shared(const SplineArgs &a, int gi, int blk, double
         // the reciprocals over the elimination's factors, which are spent
         double *rec = F + n;
         const double *d = F + 2 * n;
-        for (int r = lane; r < n; r += 64) rec[r] = 1.0 / d[r];
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        if (follow) {
+            for (int r = lane; r < n; r += 64) rec[r] = 1.0 / d[r];
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
         if (half == 0)
-            dgtsv_back(n, F, rec, sb + ls, S, [&](int i) { spline_post(&s_solved, i); });
-        spline_post(&s_solved, 0);
-        return;
+            dgtsv_back(n, F, follow ? rec : nullptr, sb + ls, S, [&](int i) {
+                if (follow) spline_post(&s_solved, i);
+            });
+        if (follow) {
+            spline_post(&s_solved, 0);
+            return;
+        }
     }
+    if (!follow) __syncthreads();
     if (ls >= nloc) return;
-    // coefficients: from the last interval down, two at a time per wave (1-3).
-    // The first half also writes the final derivatives (fill_final_derivs,
-    // interpolate.cu:242-280).
+    // coefficients: from the last interval down, two at a time per wave (1-3, or
+    // all four behind the barrier).  The half that takes the last interval also
+    // writes the final derivatives (fill_final_derivs, interpolate.cu:242-280).
     const int s = s0 + ls;
+    const int first = follow ? 1 : 0;
     double c1L = 0.0, c2L = 0.0, c3L = 0.0;
-    for (int top = n - 2 - 2 * (wv - 1); top >= 0; top -= 6) {
-        while (spline_peek(&s_solved) > max(top - 1, 0)) __builtin_amdgcn_s_sleep(1);
+    for (int top = n - 2 - 2 * (wv - first); top >= 0; top -= 2 * (4 - first)) {
+        if (follow)
+            while (spline_peek(&s_solved) > max(top - 1, 0)) __builtin_amdgcn_s_sleep(1);
         const int i = top - half;
         if (i >= 0)
             spline_emit(G, s, n, i, sb[(long)i * S + ls], sb[(long)(i + 1) * S + ls], sx[i], sx[i + 1],
                         sy[(long)i * S + ls], sy[(long)(i + 1) * S + ls], c1L, c2L, c3L);
     }
-    if (!G.dense && wv == 1 && half == 0) {
+    if (!G.dense && wv == first && half == 0) {
         const double xx = sx[n - 1] - sx[n - 2];
         const double x2 = xx * xx;
         double *out = G.out;
