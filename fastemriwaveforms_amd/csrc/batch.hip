@@ -7,7 +7,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <map>
 #include <vector>
 
 #include "batch.hpp"
@@ -85,8 +84,6 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
     // union geometry over every waveform's modes
     build_fact_plan(h_m, h_k, h_n, (int)Ksum, bp->uni);
     FactPlanHost &u = bp->uni;
-    std::map<std::pair<int, int>, int> rowmap;
-    for (int r = 0; r < u.Nr; r++) rowmap[{u.row_m[r], u.row_k[r]}] = r;
     const int ncell = u.Nr * u.Nc;
     std::vector<int> cells, ents, dstart, dmember, dcell(ncell);
     std::vector<long> sys_prefix(B + 1, 0);
@@ -113,28 +110,24 @@ void *few_batch_create(int B, const int *h_L, const int *h_K, const int *h_N, co
         d.seg_off = bp->total_intervals;
         d.tpref_off = bp->total_tpref;
         d.sys_off = (int)bp->total_systems;
-        // gather lists of this waveform on the union grid (local mode indices)
-        const int *m = h_m + mode_off, *k = h_k + mode_off, *n = h_n + mode_off;
+        // gather lists of this waveform on the union grid (local mode indices): the
+        // union plan holds every mode's cell and its mirror's (-1: m = 0)
+        const int *mc = u.mode_cell.data() + 2 * mode_off;
         std::vector<int> count(ncell + 1, 0);
-        auto cell_of = [&](int mm, int kk, int nn) { return rowmap[{mm, kk}] * u.Nc + (nn - u.n_lo); };
-        for (int q = 0; q < K; q++) {
-            count[cell_of(m[q], k[q], n[q]) + 1]++;
-            if (m[q] != 0) count[cell_of(-m[q], -k[q], -n[q]) + 1]++;
-        }
+        for (int q = 0; q < 2 * K; q++)
+            if (mc[q] >= 0) count[mc[q] + 1]++;
         std::vector<int> cs(ncell + 1, 0);
         for (int c = 0; c < ncell; c++) cs[c + 1] = cs[c] + count[c + 1];
         std::vector<int> e(cs[ncell]);
         std::vector<int> fill(cs.begin(), cs.end() - 1);
-        for (int q = 0; q < K; q++) {
-            e[fill[cell_of(m[q], k[q], n[q])]++] = 2 * q;
-            if (m[q] != 0) e[fill[cell_of(-m[q], -k[q], -n[q])]++] = 2 * q + 1;
-        }
+        for (int q = 0; q < 2 * K; q++)
+            if (mc[q] >= 0) e[fill[mc[q]]++] = q;
         // cells of the FP64 direct sum: the distinct (m, k, n) in the order of
         // their first modes, members ascending (the order of launch_cell_index)
         std::fill(dcell.begin(), dcell.end(), -1);
         std::vector<int> dsize, did(K);
         for (int q = 0; q < K; q++) {
-            int &id = dcell[cell_of(m[q], k[q], n[q])];
+            int &id = dcell[mc[2 * q]];
             if (id < 0) {
                 id = (int)dsize.size();
                 dsize.push_back(0);
