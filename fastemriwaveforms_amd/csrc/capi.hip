@@ -438,6 +438,12 @@ static int run_waveform(double2 *wave, const double *interp, const double *pt, c
 
 #define ADJ_CHUNK 2048   // samples per chunk of the mode-sum adjoint
 #define ADJ_GROUP 128    // cells per workgroup of the mode-sum adjoint
+// The modes are grouped into cells where a cell per mode makes more workgroups than
+// this: up to one per CU the time is one workgroup's whatever their number, and the
+// index only adds to it (500 modes: 158 samples 26.6 us, 38.2 grouped; 31,559 samples
+// 187 and 199; 3843 modes: 316 samples 32.4 and 61.7).  Beyond, grouping saves whole
+// rounds: 1000 modes, 31,559 samples (368 workgroups) 206 us, 327 ungrouped.
+#define ADJ_GROUP_BLOCKS 256
 
 struct AdjLayout {
     size_t segs, prefix, amp, phase, total;
@@ -850,8 +856,10 @@ int few_waveform_adjoint_async(const void *grad_wave, const double *interp_array
     a.part_phase = reinterpret_cast<double *>(ws + al.phase);
     if (K > 0 && out_len > 0) {
         // behind the parts every call needs (a workspace without it: ungrouped)
-        rc = group_modes(d_m, d_k, d_n, K, ws, workspace_bytes, al.total, a.cells, st);
-        if (rc) return rc;
+        if ((long)al.max_chunks * al.groups > ADJ_GROUP_BLOCKS) {
+            rc = group_modes(d_m, d_k, d_n, K, ws, workspace_bytes, al.total, a.cells, st);
+            if (rc) return rc;
+        }
         rc = launch_adjoint_fp64(a, (int)al.max_chunks, st);
         if (rc) return rc;
     }
