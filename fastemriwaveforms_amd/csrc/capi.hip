@@ -228,6 +228,15 @@ static int prep_check(const PrepKey &k, const char *what)
     return FEW_ERR_ARG;
 }
 
+// The samples per tile a workspace was last prepared with (0: never prepared).
+static int prep_tile(const void *ws)
+{
+    std::lock_guard<std::mutex> lk(g_prep_mu);
+    for (const PrepKey &e : g_prep)
+        if (e.ws == ws) return e.tile;
+    return 0;
+}
+
 int prep_stage(bool prepares, bool sums, const PrepKey &k, const char *what)
 {
     if (prepares) {
@@ -399,7 +408,10 @@ static int run_waveform(double2 *wave, const double *interp, const double *pt, c
         set_error("get_waveform: precision %d is not supported", precision);
         return FEW_ERR_UNSUPPORTED;
     }
-    const int tile = direct_tile(out_len, K);
+    // A sum alone takes the tiles its preparation laid out, which depend on the number
+    // of modes of that call; the sum may be of other modes.
+    int tile = direct_tile(out_len, K);
+    if (!(stage & 1) && direct_tile_ok(prep_tile(ws))) tile = prep_tile(ws);
     const PrepKey key{ws, plan, precision, tile, L, out_len};
     if (int rc = prep_stage(stage & 1, stage & 2, key, "get_waveform")) return rc;
     if (stage & 1) {
@@ -425,7 +437,7 @@ static int run_waveform(double2 *wave, const double *interp, const double *pt, c
     a.out_len = out_len;
     a.overwrite = (stage & 4) ? 1 : 0;
     const long max_blocks = ((long)out_len + tile - 1) / tile + (L - 1);
-    if (max_blocks > 0x7fffffffL) {
+    if (2 * max_blocks > 0x7fffffffL) {
         set_error("get_waveform: output too long (%d samples)", out_len);
         return FEW_ERR_LIMIT;
     }

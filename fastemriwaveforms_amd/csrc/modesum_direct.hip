@@ -335,19 +335,20 @@ __device__ __forceinline__ void direct_zero_tail(const DirectArgs &a, long block
         a.wave[i] = make_double2(0.0, 0.0);
 }
 
+// PER: workgroups per tile of the interval plan, a part of it each.
 // Four waves per SIMD: 128 registers, of which the four-sample form spills 51 (208 B
 // of scratch), most of them around the repetition with the library sincos.
-template <int SPT>
+template <int SPT, int PER>
 __global__ __launch_bounds__(256, 4) void direct_fp64_kernel(DirectArgs a)
 {
     __shared__ DirectLds sh;
-    const int b = blockIdx.x;
+    const int b = blockIdx.x / PER;
     const int total = a.prefix[a.nseg];
     if (b < total) {
         const int j = find_segment(a.prefix, a.nseg, b);
-        direct_fp64_tile<SPT>(a, j, b - a.prefix[j], sh);
+        direct_fp64_tile<SPT>(a, j, PER * (b - a.prefix[j]) + blockIdx.x % PER, sh);
     }
-    if (a.overwrite) direct_zero_tail(a, b, gridDim.x);
+    if (a.overwrite) direct_zero_tail(a, blockIdx.x, gridDim.x);
 }
 
 template <int SPT>
@@ -479,7 +480,7 @@ int launch_plan(const PlanArgs &p, hipStream_t stream)
 // of them per mode.  Added to an output of 94,675 samples 1 / 8 / 12 / 20 modes take
 // 8.1 / 10.0 / 10.9 / 13.0 us (11.1 / 12.1 / 12.7 / 13.9 with four waves on the same
 // samples), 9468 samples 7.9 / 9.5 / 10.5 / 12.6 us (7.7 / 8.0 / 8.0 / 8.6).
-bool direct_few(long out_len, int K) { return K <= DIRECT_FEW && out_len >= 4096L * K; }
+static bool direct_few(long out_len, int K) { return K <= DIRECT_FEW && out_len >= 4096L * K; }
 
 // Otherwise, below 2^17 samples the four-sample tiles are too few to fill the chip:
 // 63,116 samples of the full set take 128 us with one sample per lane and 183 us
@@ -493,13 +494,16 @@ int direct_tile(long out_len, int K)
 int launch_direct_fp64(const DirectArgs &a, int tile, int max_blocks, hipStream_t stream)
 {
     if (max_blocks <= 0) return FEW_OK;
-    const dim3 grid(max_blocks);
-    if (tile == DIRECT_FEW_TILE)
-        hipLaunchKernelGGL(direct_few_kernel<DIRECT_FEW_TILE / 256>, grid, dim3(256), 0, stream, a);
+    const dim3 grid(max_blocks), block(256);
+    if (tile == DIRECT_FEW_TILE && a.K <= DIRECT_FEW)
+        hipLaunchKernelGGL(direct_few_kernel<DIRECT_FEW_TILE / 256>, grid, block, 0, stream, a);
+    else if (tile == DIRECT_FEW_TILE)  // laid out for few modes, summed for many
+        hipLaunchKernelGGL((direct_fp64_kernel<DIRECT_SPT, DIRECT_FEW_TILE / DIRECT_TILE>),
+                           dim3(max_blocks * (DIRECT_FEW_TILE / DIRECT_TILE)), block, 0, stream, a);
     else if (tile == DIRECT_TILE)
-        hipLaunchKernelGGL(direct_fp64_kernel<DIRECT_SPT>, grid, dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((direct_fp64_kernel<DIRECT_SPT, 1>), grid, block, 0, stream, a);
     else
-        hipLaunchKernelGGL(direct_fp64_kernel<1>, grid, dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((direct_fp64_kernel<1, 1>), grid, block, 0, stream, a);
     FEW_HIP(hipGetLastError());
     return FEW_OK;
 }

@@ -203,10 +203,13 @@ constexpr int DIRECT_TILE = 64 * DIRECT_SPT;
 // samples (a batch keeps DIRECT_TILE).
 constexpr int DIRECT_FEW = 16;
 constexpr int DIRECT_FEW_TILE = 512;
-// Whether the FP64 direct sum of K modes and out_len samples runs that way.
-bool direct_few(long out_len, int K);
 // Samples per tile of the FP64 direct sum of K modes for an output of out_len samples.
 int direct_tile(long out_len, int K);
+// Whether launch_direct_fp64 takes tiles of this many samples (for any set of modes).
+constexpr bool direct_tile_ok(int tile)
+{
+    return tile == 64 || tile == DIRECT_TILE || tile == DIRECT_FEW_TILE;
+}
 int launch_direct_fp64(const DirectArgs &a, int tile, int max_blocks, hipStream_t stream);
 
 }  // namespace few

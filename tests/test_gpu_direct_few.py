@@ -78,3 +78,31 @@ def test_batch(gpu):
     b.run("fp64")
     for i, inp in enumerate(inputs):
         np.testing.assert_array_equal(b.waveform(i).cpu().numpy(), _run(inp))
+
+
+@pytest.mark.parametrize("prepared,summed", [(3, 200), (200, 3), (16, 17), (5, 6)])
+@pytest.mark.parametrize("num", [70001, 140000])
+def test_sum_of_other_modes_than_prepared(gpu, prepared, summed, num):
+    """The interval plan does not depend on the modes: a sum may follow the preparing
+    call of another set, whichever way either runs, and another precision's stays
+    refused."""
+    from fastemriwaveforms_amd._lib import lib
+    from fastemriwaveforms_amd.pipeline import ModeSumProblem, _stream
+    a, b = _input(prepared, num), _input(summed, num)
+    pa, pb = ModeSumProblem(a), ModeSumProblem(dataclasses.replace(b, t=a.t, dense=a.dense))
+    pb.build_splines()
+
+    def call(p, ws, precision, stage):
+        return lib().few_get_waveform_plan_async(
+            p.wave.data_ptr(), p.interp.data_ptr(), p.t.data_ptr(), p.pcoef.data_ptr(), None,
+            p.m.data_ptr(), p.k.data_ptr(), p.n.data_ptr(), p.L, p.N, p.K, p.ylm.data_ptr(), p.dt,
+            p.t.data_ptr(), precision, 0, stage, ws.data_ptr(), ws.numel(), _stream())
+
+    want = pb.run("fp64").cpu().numpy()
+    ws = pb.ws if pb.ws.numel() >= pa.ws.numel() else pa.ws
+    pb.wave.fill_(5.0)
+    assert call(pa, ws, 0, 1) == 0, lib().few_last_error()
+    assert call(pb, ws, 0, 6) == 0, lib().few_last_error()
+    np.testing.assert_array_equal(pb.wave.cpu().numpy(), want)
+    pb.mode_sum("mixed16", 1)
+    assert call(pb, pb.ws, 0, 6) != 0
