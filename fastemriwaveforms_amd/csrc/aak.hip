@@ -9,10 +9,9 @@
 // The Bessel functions are the Numerical Recipes routines the reference's CPU
 // branch uses (rational / asymptotic J0, J1; Miller's backward recurrence for
 // J_n below its order), restated here so the device result follows the CPU
-// reference rather than a library jn.  aak_sample is the reference's arithmetic
-// in its order with contraction off, the cos and sin of one argument taken with
-// one sincos call (as an optimising compiler merges them); the kernel runs
-// aak_sample_fast, the same quantities with fewer operations.
+// reference rather than a library jn.  aak_sample_fast forms the reference's
+// quantities with fewer operations, with contraction off and the cos and sin of one
+// argument taken with one sincos call (as an optimising compiler merges them).
 //
 // Work layout: a one-wave planning kernel turns the knot times into sample
 // ranges with the reference's rule (gpuAAK.cu:458-483); the sum kernel runs
@@ -457,129 +456,8 @@ __host__ __device__ inline AakGeom aak_geom(const AakArgs &a)
     return g;
 }
 
-// One output sample i of segment j (gpuAAK.cu:270-451); sc[p][c] are the
-// segment's dense coefficients.  Returns hI - i hII, by the reference's
-// operations one for one (the host tests' form; the kernel's is below).
-__host__ __device__ inline double2 aak_sample(const AakArgs &a, const double (*sc)[8], double start_t,
-                                              double segwidth, long i)
-{
-    const AakGeom G = aak_geom(a);
-    const double phiS = a.phiS, phiK = a.phiK;
-    const double cosqS = G.cosqS, sinqS = G.sinqS, cosqK = G.cosqK, sinqK = G.sinqK;
-    const double cosphiK = G.cosphiK, sinphiK = G.sinphiK, cosphiS = G.cosphiS, sinphiS = G.sinphiS;
-    const double cosdphi = G.cosdphi, sindphi = G.sindphi;
-    const double halfsqrt3 = sqrt(3.) / 2.;
-    const double mu_sec = a.mu * AAK_MTSUN_SI;
-    const double zeta = mu_sec / a.dist / AAK_GPCINSEC;
-    const double t = a.dt * i;
-    const double s = (t - start_t) / segwidth;
-    const double s1 = (1.0 - s);
-    const double s2 = s * s, s3 = s * s2, s4 = s * s3, s5 = s * s4, s6 = s * s5;
-    const double e = aak_dense(sc[1], s, s1);
-    const double Y = aak_dense(sc[2], s, s1);
-    const double Phi_phi = aak_dense(sc[3], s, s1);
-    const double Phi_theta = aak_dense(sc[4], s, s1);
-    const double Phi_r = aak_dense(sc[5], s, s1);
-    const double OmegaPhi = aak_dense_dot(sc[3], s, s2, s3, s4, s5, s6) / segwidth;
-    const double OmegaTheta = aak_dense_dot(sc[4], s, s2, s3, s4, s5, s6) / segwidth;
-    const double OmegaR = aak_dense_dot(sc[5], s, s2, s3, s4, s5, s6) / segwidth;
-    const double Phi = Phi_r;
-    const double gim = Phi_theta - Phi_r;
-    const double alp = Phi_phi - Phi_theta;
-    const double nu = OmegaR / (2. * M_PI);
-    const double gimdot = OmegaTheta - OmegaR;
-    const double lam = acos(Y);
-    double coslam, sinlam, cosalp, sinalp;
-    sincos(lam, &sinlam, &coslam);
-    sincos(alp, &sinalp, &cosalp);
-    const double cosqL = cosqK * coslam + sinqK * sinlam * cosalp;
-    const double sinqL = sqrt(1. - cosqL * cosqL);
-    const double phiLup = sinqK * sinphiK * coslam - cosphiK * sinlam * sinalp - cosqK * sinphiK * sinlam * cosalp;
-    const double phiLdown = sinqK * cosphiK * coslam + sinphiK * sinlam * sinalp - cosqK * cosphiK * sinlam * cosalp;
-    const double phiL = atan2(phiLup, phiLdown);
-    const double Ldotn = cosqL * cosqS + sinqL * sinqS * cos(phiL - phiS);
-    const double Ldotn2 = Ldotn * Ldotn;
-    const double Sdotn = cosqK * cosqS + sinqK * sinqS * cosdphi;
-    double beta;
-    if (a.S_phys == 0.0 || lam < 1e-10 || lam > (M_PI - 1e-10)) {
-        beta = 0.0;
-    } else {
-        const double betaup = -Sdotn + coslam * Ldotn;
-        const double betadown = sinqS * sindphi * sinlam * cosalp + (cosqK * Sdotn - cosqS) / sinqK * sinlam * sinalp;
-        beta = atan2(betaup, betadown);
-    }
-    const double gam = 2. * (gim + beta);
-    double cos2gam, sin2gam;
-    sincos(gam, &sin2gam, &cos2gam);
-    double cosorbphs = 0, FplusI, FcrosI, FplusII, FcrosII;
-    if (a.mich) {
-        const double orbphs = 2. * M_PI * t / AAK_YRSID_SI;
-        double sinorbphs, sinorb, cosorb;
-        sincos(orbphs - phiS, &sinorbphs, &cosorbphs);
-        sincos(orbphs, &sinorb, &cosorb);
-        const double cosq = .5 * cosqS - halfsqrt3 * sinqS * cosorbphs;
-        const double phiw = orbphs + atan2(halfsqrt3 * cosqS + .5 * sinqS * cosorbphs, sinqS * sinorbphs);
-        const double psiup = .5 * cosqK - halfsqrt3 * sinqK * cos(orbphs - phiK) - cosq * (cosqK * cosqS + sinqK * sinqS * cosdphi);
-        const double psidown = .5 * sinqK * sinqS * sindphi - halfsqrt3 * cosorb * (cosqK * sinqS * sinphiS - cosqS * sinqK * sinphiK) - halfsqrt3 * sinorb * (cosqS * sinqK * cosphiK - cosqK * sinqS * cosphiS);
-        const double psi = atan2(psiup, psidown);
-        const double cosq1 = .5 * (1. + cosq * cosq);
-        double cos2phi, sin2phi, cos2psi, sin2psi;
-        sincos(2. * phiw, &sin2phi, &cos2phi);
-        sincos(2. * psi, &sin2psi, &cos2psi);
-        FplusI = cosq1 * cos2phi * cos2psi - cosq * sin2phi * sin2psi;
-        FcrosI = cosq1 * cos2phi * sin2psi + cosq * sin2phi * cos2psi;
-        FplusII = cosq1 * sin2phi * cos2psi + cosq * cos2phi * sin2psi;
-        FcrosII = cosq1 * sin2phi * sin2psi - cosq * cos2phi * cos2psi;
-    } else {
-        FplusI = 1.0;
-        FcrosI = 0.0;
-        FplusII = 0.0;
-        FcrosII = 1.0;
-    }
-    const double Amp = pow(fabs(OmegaPhi) * a.M_phys * AAK_MTSUN_SI, 2. / 3.) * zeta;
-    double rot[4];
-    aak_rot_coeff(rot, sinlam, coslam, sinqS, cosqS, sinphiS, cosphiS, sinqK, cosqK, sinphiK, cosphiK,
-                  sinalp, cosalp);
-    double hItemp = 0.0, hIItemp = 0.0;
-    const double sq1e = sqrt(1 - e * e);
-    for (int n = 1; n <= a.nmodes; n++) {
-        double nPhi;
-        if (a.mich) {
-            const double fn = n * nu + gimdot / M_PI;
-            const double Doppler = 2. * M_PI * fn * AAK_AUSEC * sinqS * cosorbphs;
-            nPhi = n * Phi + Doppler;
-        } else {
-            nPhi = n * Phi;
-        }
-        const double ne = n * e;
-        double Jv[5];
-        nr_jn5(n - 2, ne, Jv);
-        const double J0 = (n == 1) ? -1.0 * Jv[2] : Jv[0];
-        const double J1 = Jv[1], J2 = Jv[2], J3 = Jv[3], J4 = Jv[4];
-        double sn, cn;
-        sincos(nPhi, &sn, &cn);
-        const double aa = -n * Amp * (J0 - 2. * e * J1 + 2. / n * J2 + 2. * e * J3 - J4) * cn;
-        const double bb = -n * Amp * sq1e * (J0 - 2. * J2 + J4) * sn;
-        const double cc = 2. * Amp * J2 * cn;
-        const double Aplus0 = -(1. + Ldotn2) * (aa * cos2gam - bb * sin2gam) + cc * (1 - Ldotn2);
-        const double Acros0 = 2. * Ldotn * (bb * cos2gam + aa * sin2gam);
-        const double Aplus = Aplus0 * rot[0] + Acros0 * rot[1];
-        const double Acros = Aplus0 * rot[2] + Acros0 * rot[3];
-        double hnI, hnII;
-        if (a.mich) {
-            hnI = halfsqrt3 * (FplusI * Aplus + FcrosI * Acros);
-            hnII = halfsqrt3 * (FplusII * Aplus + FcrosII * Acros);
-        } else {
-            hnI = FplusI * Aplus + FcrosI * Acros;
-            hnII = FplusII * Aplus + FcrosII * Acros;
-        }
-        hItemp += hnI;
-        hIItemp += hnII;
-    }
-    return make_double2(hItemp, -hIItemp);
-}
-
-// aak_sample in the kernel's form.  What the phases of 1e5-1e6 rad pass through
+// One output sample i of segment j (gpuAAK.cu:270-451); sc[p][c] are the segment's
+// dense coefficients.  Returns hI - i hII.  What the phases of 1e5-1e6 rad pass through
 // (the splines, gim + beta, n Phi + Doppler) is the same operations, as an ulp
 // there is 1e-11 and more; the rest is the same quantities with fewer of them:
 //   * the harmonics enter h through three sums over n, sum a_n, b_n and c_n,
@@ -703,27 +581,9 @@ __host__ __device__ inline double2 aak_sample_fast(const AakArgs &a, const AakGe
     return make_double2(FplusI * Aplus + FcrosI * Acros, -(FplusII * Aplus + FcrosII * Acros));
 }
 
-// gpuAAK.cu:458-483: start index of every segment and the number of knots
-// used; segments stop at the last knot when none reaches the end (the
-// reference then reads past its arrays).
-__host__ __device__ inline int aak_plan(const double *h_t, int L, double dt, int out_len, int *st)
-{
-    const double T = (out_len - 1) * dt;
-    st[0] = 0;
-    int i;
-    for (i = 1; i < L; i++) {
-        const double t = h_t[i];
-        if (t < T) {
-            st[i] = (int)ceil(t / dt);
-        } else {
-            st[i] = out_len;
-            break;
-        }
-    }
-    return i < L ? i + 1 : L;
-}
-
-// aak_plan, one knot per lane: knots up to the first at or past the end.
+// gpuAAK.cu:458-483: start index of every segment and the number of knots used;
+// segments stop at the last knot when none reaches the end (the reference then
+// reads past its arrays).  One knot per lane, up to the first at or past the end.
 __global__ __launch_bounds__(64) void aak_plan_kernel(AakArgs a)
 {
     const double T = (a.out_len - 1) * a.dt;

@@ -61,15 +61,6 @@ __host__ __device__ inline int amp_interval(const double *t, int n, int k, doubl
     return l - k1;
 }
 
-__host__ __device__ inline void amp_point_basis(const double *tx, int nx, const double *ty, int ny,
-                                                int kx, int ky, double x, double y, double *b)
-{
-    const int lx = amp_interval(tx, nx, kx, x, b + 2);
-    const int ly = amp_interval(ty, ny, ky, y, b + 8);
-    b[0] = (double)lx;
-    b[1] = (double)ly;
-}
-
 // fpbisp's sum (AmpInterp2D.cu:73-83) for one coefficient set.
 __host__ __device__ inline double amp_sum(const double *c, int nky1, int kx, int ky, const double *b)
 {

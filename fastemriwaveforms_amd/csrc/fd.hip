@@ -26,13 +26,13 @@
 // segment) items are flattened, their in-range bin counts prefix-summed on
 // the device, and a persistent grid walks the flattened bins.
 //
-// The kernels evaluate fd_bin_fast, a shorter form of the reference's bin,
-// fd_bin, which the host tests hold it against.  fd_bin's complex arithmetic
-// follows gcmplx::complex (src/few/cutils/cuda_complex.hpp,
-// the libc++ <complex> algorithms) operation for operation, on the device's
-// FP64 libm, with contraction off in the whole file; the products keep their
-// C99 Annex G NaN recovery.  cos and sin of one argument are taken with one
-// sincos call, as an optimising compiler emits for gcmplx::exp / polar.
+// The kernels evaluate fd_bin_fast, a shorter form of the reference's bin
+// (interpolate.cu:1240-1500), with contraction off in the whole file.  The complex
+// arithmetic of its rare branches and constants follows gcmplx::complex
+// (src/few/cutils/cuda_complex.hpp, the libc++ <complex> algorithms) operation for
+// operation, on the device's FP64 libm; the products keep their C99 Annex G NaN
+// recovery.  cos and sin of one argument are taken with one sincos call, as an
+// optimising compiler emits for gcmplx::exp / polar.
 #include <math.h>
 
 #include <algorithm>
@@ -258,74 +258,9 @@ __host__ __device__ inline fcx fd_spa(double x, const FdSpaConst &kc)
     return fcx_mul(pref, ser);
 }
 
-// cube_roots (interpolate.cu:1113-1134): Cardano with the principal complex
-// cube root; xi = (-1 + sqrt(-3)) / 2 is passed in (computed once per thread).
-__host__ __device__ inline void fd_cube_roots(double a, double b, double c, double d, fcx xi,
-                                              double out[3])
-{
-#pragma clang fp contract(off)
-    const double b2 = b * b;
-    const double b3 = b2 * b;
-    const double a2 = a * a;
-    const double D0 = (b2 - 3 * a * c);
-    const double D1 = (2 * b3 - 9 * a * b * c + 27 * a2 * d);
-    const fcx sq = fcx_sqrt(fcx_make(D1 * D1 - 4 * (D0 * D0 * D0), 0.0));
-    const fcx C = fcx_pow(fcx_divr(fcx_addr(D1, sq), 2.), 1. / 3.);
-    const double pre = -(1. / (3 * a));
-    const fcx xiC = fcx_mul(xi, C);
-    const fcx xixiC = fcx_mul(fcx_mul(xi, xi), C);
-    out[0] = fcx_scale(fcx_add(fcx_addr(b, C), fcx_rdiv(D0, C)), pre).re;
-    out[1] = fcx_scale(fcx_add(fcx_addr(b, xiC), fcx_rdiv(D0, xiC)), pre).re;
-    out[2] = fcx_scale(fcx_add(fcx_addr(b, xixiC), fcx_rdiv(D0, xixiC)), pre).re;
-}
-
 __host__ __device__ inline fcx fd_xi()
 {
     return fcx_divr(fcx_addr(-1., fcx_sqrt(fcx_make(-3., 0.0))), 2.);
-}
-
-// Everything one (mode, segment) item reads (interpolate.cu:1240-1345).
-struct FdItem {
-    double ar[4], ai[4];          // amplitude cubic, Re and Im
-    double pp[8], pt[8], pr[8];   // dense-output phases
-    double F0, F1, F2, F3;        // mode-frequency cubic
-    double t0, t1, pt0, pw;       // segment bounds, phase segment start and width
-    double mm, kk, nn;
-    fcx yp, ym;
-};
-
-__host__ __device__ inline void fd_load_item(const FdArgs &a, int q, int j, FdItem &it)
-{
-#pragma clang fp contract(off)
-    const long nb = (2L * a.K + 3) * a.L;
-    const long np = (long)(a.L - 1) * 3;
-    double fph[4], fth[4], frr[4];
-    for (int c = 0; c < 4; c++) {
-        it.ar[c] = a.interp[c * nb + (long)q * a.L + j];
-        it.ai[c] = a.interp[c * nb + (long)(a.K + q) * a.L + j];
-        fph[c] = a.interp[c * nb + (long)(2 * a.K) * a.L + j];
-        fth[c] = a.interp[c * nb + (long)(2 * a.K + 1) * a.L + j];
-        frr[c] = a.interp[c * nb + (long)(2 * a.K + 2) * a.L + j];
-    }
-    for (int c = 0; c < 8; c++) {
-        it.pp[c] = a.pcoef[c * np + j];
-        it.pt[c] = a.pcoef[c * np + (a.L - 1) + j];
-        it.pr[c] = a.pcoef[c * np + 2 * (a.L - 1) + j];
-    }
-    const int m = a.m[q], k = a.k[q], n = a.n[q];
-    it.mm = m;
-    it.kk = k;
-    it.nn = n;
-    it.F0 = m * fph[0] + k * fth[0] + n * frr[0];
-    it.F1 = m * fph[1] + k * fth[1] + n * frr[1];
-    it.F2 = m * fph[2] + k * fth[2] + n * frr[2];
-    it.F3 = m * fph[3] + k * fth[3] + n * frr[3];
-    it.t0 = a.t_knots[j];
-    it.t1 = a.t_knots[j + 1];
-    it.pt0 = a.phase_t[j];
-    it.pw = a.phase_t[j + 1] - a.phase_t[j];
-    it.yp = fcx_make(a.ylm[q].x, a.ylm[q].y);
-    it.ym = fcx_make(a.ylm[a.K + q].x, a.ylm[a.K + q].y);
 }
 
 __host__ __device__ inline double fd_phase(const double *r, double s, double s1)
@@ -334,80 +269,21 @@ __host__ __device__ inline double fd_phase(const double *r, double s, double s1)
     return r[0] + s * (r[1] + s1 * (r[2] + s * (r[3] + s1 * (r[4] + s * (r[5] + s1 * (r[6] + s * r[7]))))));
 }
 
-__host__ __device__ inline double fd_fdot(const double *r, double s, double s2, double s3,
-                                          double s4, double s5, double w2)
-{
-#pragma clang fp contract(off)
-    return (-2. * r[2] + r[3] * (2. - 6. * s) + r[4] * (2. - 12. * s + 12. * s2) +
-            r[5] * (6. * s - 24. * s2 + 20. * s3) + r[6] * (6. * s - 36. * s2 + 60. * s3 - 30. * s4) +
-            r[7] * (12. * s2 - 60. * s3 + 90. * s4 - 42. * s5)) /
-           (2. * M_PI * w2);
-}
-
-__host__ __device__ inline double fd_fddot(const double *r, double s, double s2, double s3,
-                                           double s4, double w3)
-{
-#pragma clang fp contract(off)
-    return (-6. * r[3] + r[4] * (-12. + 24. * s) + r[5] * (6. - 48. * s + 60. * s2) +
-            r[6] * (6. - 72. * s + 180. * s2 - 120. * s3) +
-            r[7] * (24. * s - 180. * s2 + 360. * s3 - 210. * s4)) /
-           (2. * M_PI * w3);
-}
-
-// The contributions of bin i of an item: one per root inside the segment
-// (up to three), each the +f term and the -f (conjugate) term, handed to
-// emit(plus, minus) in root order.
-template <class Emit>
-__host__ __device__ inline void fd_bin(const FdItem &it, double f, fcx xi, const FdSpaConst &kc,
-                                       Emit emit)
-{
-#pragma clang fp contract(off)
-    double roots[3];
-    fd_cube_roots(it.F3, it.F2, it.F1, (it.F0 - f), xi, roots);
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        const double root = roots[r];
-        const double t = it.t0 + root;
-        if (!((t < it.t1) && (t >= it.t0))) continue;
-        const double x = root, x2 = x * x, x3 = x * x2;
-        const double Are = it.ar[0] + it.ar[1] * x + it.ar[2] * x2 + it.ar[3] * x3;
-        const double Aim = it.ai[0] + it.ai[1] * x + it.ai[2] * x2 + it.ai[3] * x3;
-        const double s = (t - it.pt0) / it.pw;
-        const double s1 = 1.0 - s;
-        const double s2 = s * s, s3 = s * s2, s4 = s * s3, s5 = s * s4;
-        const double w2 = it.pw * it.pw;
-        const double w3 = it.pw * w2;
-        const double phase = it.mm * fd_phase(it.pp, s, s1) + it.kk * fd_phase(it.pt, s, s1) +
-                             it.nn * fd_phase(it.pr, s, s1);
-        const double fdot = it.mm * fd_fdot(it.pp, s, s2, s3, s4, s5, w2) +
-                            it.kk * fd_fdot(it.pt, s, s2, s3, s4, s5, w2) +
-                            it.nn * fd_fdot(it.pr, s, s2, s3, s4, s5, w2);
-        const double fddot = it.mm * fd_fddot(it.pp, s, s2, s3, s4, w3) +
-                             it.kk * fd_fddot(it.pt, s, s2, s3, s4, w3) +
-                             it.nn * fd_fddot(it.pr, s, s2, s3, s4, w3);
-        const double targ = 2. * M_PI * fdot * fdot * fdot / (3. * fddot * fddot);
-        const double pre = -1.0 * fdot / fabs(fddot) * 2. / sqrt(3.);
-        const fcx amp2 = fcx_div(fcx_scale(fd_spa(targ, kc), pre), fcx_sqrt(fcx_make(targ, 0.0)));
-        const fcx ph = fcx_exp(fcx_scale(fcx_make(0.0, 1.0), 2. * M_PI * f * t - phase));
-        const fcx te = fcx_mul(fcx_mul(fcx_make(Are, Aim), amp2), ph);
-        emit(fcx_mul(it.yp, te), fcx_mul(it.ym, fcx_make(te.re, -te.im)));
-    }
-}
-
 // ---------------------------------------------------------------- fast form
 // What the kernels evaluate: the same roots, phase and stationary-phase factor
-// as fd_bin, without the complex library calls on numbers that are real or
-// purely imaginary and with everything that depends on the segment alone formed
-// once per segment.  fd_bin, the reference's operations one for one, spends
-// ~2300 instructions per bin, this form ~600.  What keeps the two close:
+// as the reference's bin, without the complex library calls on numbers that are
+// real or purely imaginary and with everything that depends on the segment alone
+// formed once per segment.  The reference's operations one for one take ~2300
+// instructions per bin, this form ~600.  What keeps the two close:
 //   * the time of a root decides 2 pi f t - phase, of which an ulp of t is
-//     ~1e-11 at 1e5 rad, so the roots are fd_cube_roots' own values, all but a
-//     few bit for bit: the same operations, only that the discriminant is real
+//     ~1e-11 at 1e5 rad, so the roots are cube_roots' (interpolate.cu:1113-1134) own
+//     values, 98 % of them bit for bit: Cardano's formula with the principal complex
+//     cube root in the same operations, only that the discriminant is real
 //     (its square root and, unless it is negative, the cube root need no hypot,
 //     atan2 or sincos), that |C|^2 >= 1e-216 needs no scaling in D0 / C, and
 //     that roots outside the segment (by a quotient shared by the three, with
 //     a margin) are dropped before theirs is formed;
-//   * s and the phases are fd_bin's values (s by a correctly rounded quotient);
+//   * s and the phases are the reference's values (s by a correctly rounded quotient);
 //   * the frequency's derivatives enter the amplitude only, so they are
 //     polynomials in s with fused steps.
 
@@ -458,7 +334,7 @@ __host__ __device__ inline void fd_load_seg(const FdArgs &a, int q, int j, FdSeg
     const double F1 = m * fph[1] + k * fth[1] + n * frr[1];
     const double F2 = m * fph[2] + k * fth[2] + n * frr[2];
     const double F3 = m * fph[3] + k * fth[3] + n * frr[3];
-    // fd_cube_roots(F3, F2, F1, F0 - f), what does not depend on f
+    // the cubic (F3, F2, F1, F0 - f), what does not depend on f
     const double b2 = F2 * F2;
     const double b3 = b2 * F2;
     const double a2 = F3 * F3;
@@ -473,7 +349,8 @@ __host__ __device__ inline void fd_load_seg(const FdArgs &a, int q, int j, FdSeg
     it.pt0 = a.phase_t[j];
     it.pw = a.phase_t[j + 1] - a.phase_t[j];
     it.rpw = 1.0 / it.pw;
-    // fd_fdot's terms by powers of s; fd_fddot is their derivative over pw
+    // the second derivative of the phases over 2 pi by powers of s (interpolate.cu's
+    // fdot), then its derivative over pw (fddot)
     const double w = 1.0 / (2. * M_PI * (it.pw * it.pw));
     it.f[0] = (2. * (r[3] - r[2] + r[4])) * w;
     it.f[1] = (6. * (r[5] + r[6] - r[3]) - 12. * r[4]) * w;
@@ -493,7 +370,7 @@ __host__ __device__ __attribute__((noinline)) fcx fd_sincos_any(double x)
     sincos(x, &r.im, &r.re);
     return r;
 }
-// pre SPA(x) / sqrt(x) from the two derivatives, as fd_bin forms it
+// pre SPA(x) / sqrt(x) from the two derivatives, as the reference forms it
 __host__ __device__ __attribute__((noinline)) fcx fd_amp_any(double fdot, double fddot,
                                                             const FdSpaConst kc)
 {
@@ -554,7 +431,7 @@ __host__ __device__ inline FdRootConst fd_root_const()
     return k;
 }
 
-// C, C xi and C xi^2 of the cubic at d = F0 - f (fd_cube_roots).
+// C, C xi and C xi^2 of the cubic at d = F0 - f, xi = (-1 + sqrt(-3)) / 2.
 __host__ __device__ inline void fd_cube_c(const FdSeg &it, double d, const FdRootConst &k, fcx (&C)[3])
 {
     const double D1 = (it.D1c + it.a27 * d);
@@ -644,12 +521,6 @@ __host__ __device__ inline void fd_cell_add(double a_re, double a_im, double2 yp
     cp.im += yp.x * a_im + yp.y * a_re;
     cm.re += ym.x * a_re + ym.y * a_im;
     cm.im += ym.y * a_re - ym.x * a_im;
-}
-
-__host__ __device__ inline int fd_minus_index(int zero_index, int i)
-{
-    const int diff = abs(zero_index - i);
-    return (i < zero_index) ? zero_index + diff : zero_index - diff;
 }
 
 // In-range bins of item (q, j): [max(start, 0), min(end, Nf - 1)].

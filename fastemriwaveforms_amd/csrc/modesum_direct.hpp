@@ -114,13 +114,6 @@ __host__ __device__ inline void sample_state(double dt, int i, double h_t, doubl
     st.Pr = dense_phase(rr, s, s1);
 }
 
-struct ModeCoef {
-    double ry, rc1, rc2, rc3;     // real-part cubic
-    double iy, ic1, ic2, ic3;     // imaginary-part cubic
-    double yp_re, yp_im, ym_re, ym_im;
-    double m, k, n;
-};
-
 // m*Phi_phi + k*Phi_theta + n*Phi_r rounded exactly as the oracle
 // (interpolate.cu:662); contraction off.
 __host__ __device__ inline double mode_phase(double m, double Pp, double k, double Pt, double n,
@@ -130,32 +123,9 @@ __host__ __device__ inline double mode_phase(double m, double Pp, double k, doub
     return m * Pp + k * Pt + n * Pr;
 }
 
-// One mode's contribution at one sample (interpolate.cu:647-684):
-//   P = exp(-i*phase) * A(x);  tr += [m != 0] conj(P) Y- ;  tr += P Y+
-__host__ __device__ inline void mode_term_fp64(const ModeCoef &c, double x, double x2, double x3,
-                                               double Pp, double Pt, double Pr, double &tr_re,
-                                               double &tr_im)
-{
-    const double phase = mode_phase(c.m, Pp, c.k, Pt, c.n, Pr);
-    double e_im, e_re;
-    if (!sincos_cw(-phase, e_im, e_re)) sincos(-phase, &e_im, &e_re);
-    const double a_re = c.ry + c.rc1 * x + c.rc2 * x2 + c.rc3 * x3;
-    const double a_im = c.iy + c.ic1 * x + c.ic2 * x2 + c.ic3 * x3;
-    const double p_re = e_re * a_re - e_im * a_im;
-    const double p_im = e_re * a_im + e_im * a_re;
-    const double tp_re = p_re * c.yp_re - p_im * c.yp_im;
-    const double tp_im = p_re * c.yp_im + p_im * c.yp_re;
-    double tm_re = 0.0, tm_im = 0.0;
-    if (c.m != 0.0) {
-        tm_re = p_re * c.ym_re + p_im * c.ym_im;
-        tm_im = p_re * c.ym_im - p_im * c.ym_re;
-    }
-    tr_re = tr_re + tm_re + tp_re;
-    tr_im = tr_im + tm_im + tp_im;
-}
-
-// The same contribution for all modes of one cell (one phase): with the cubics
-// C+ = sum Y+ A and C- = sum Y- conj(A) (m != 0) of its members,
+// The contribution of all modes of one cell (one phase) at a sample, the sum of
+// Y+ P + [m != 0] Y- conj(P) with P = exp(-i phase) A (interpolate.cu:647-684): with
+// the cubics C+ = sum Y+ A and C- = sum Y- conj(A) (m != 0) of its members,
 //   C+ exp(-i phase) + C- exp(+i phase)
 //     = (P cos + Q sin) + i (R cos + S sin),
 //   P = Re C+ + Re C-, Q = Im C+ - Im C-, R = Im C+ + Im C-, S = Re C- - Re C+.

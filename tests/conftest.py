@@ -21,7 +21,7 @@ CSRC = os.path.join(ROOT, "fastemriwaveforms_amd", "csrc")
 
 def build_twin() -> str:
     """Compile the host twin of the kernel sources (hipcc, host code exercised on the CPU)."""
-    srcs = [TWIN_SRC] + [os.path.join(CSRC, f) for f in os.listdir(CSRC)]
+    srcs = [TWIN_SRC, os.path.join(ROOT, "tests", "twin_reference.hpp")] + [os.path.join(CSRC, f) for f in os.listdir(CSRC)]
     if os.path.exists(TWIN_LIB) and os.path.getmtime(TWIN_LIB) >= max(map(os.path.getmtime, srcs)):
         return TWIN_LIB
     os.makedirs(os.path.dirname(TWIN_LIB), exist_ok=True)

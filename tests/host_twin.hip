@@ -3,9 +3,11 @@
 // Compiles the product's kernel sources and runs their host-callable
 // per-system / per-sample routines on the CPU, so the CPU test suite can
 // check the exact code the GPU runs (spline recurrence, dense-output phase,
-// the direct mode term, the interval planning rule) against the oracle
+// the direct cell term, the interval planning rule) against the oracle
 // without a GPU.  Only the orchestration (tiling, LDS staging, launch
-// geometry) is left to the GPU tests.
+// geometry) is left to the GPU tests.  Where a kernel evaluates a shorter form
+// than the reference's operations, those stand in twin_reference.hpp and both
+// are run here.
 
 #include <stdarg.h>
 #include <stdio.h>
@@ -20,6 +22,7 @@
 #include "aak.hip"
 #include "modesum_direct.hpp"
 #include "few_math.hpp"
+#include "twin_reference.hpp"
 
 namespace few {
 static char g_twin_err[512];
@@ -108,7 +111,64 @@ int twin_plan(const double *h_t, int L, double dt, int out_len, int *starts, int
     return used;
 }
 
-// Direct FP64 mode sum at chosen samples with the kernel's per-mode code.
+// The interval of sample i, and its state.
+static int twin_sample(const double *h_t, const double *pt, const double *pcoef, int L, double dt,
+                       const std::vector<int> &st, const std::vector<int> &en, int i, SampleState &ss)
+{
+    for (int j = 0; j < L - 1; j++) {
+        if (i < st[j] || i >= en[j]) continue;
+        const long np = (long)(L - 1) * 3;
+        double r[3][8];
+        for (int p = 0; p < 3; p++)
+            for (int c = 0; c < 8; c++) r[p][c] = pcoef[c * np + (long)j * 3 + p];
+        sample_state(dt, i, h_t[j], pt[j], pt[j + 1] - pt[j], r[0], r[1], r[2], ss);
+        return j;
+    }
+    return -1;
+}
+
+// The FP64 sum over cells as the kernels form it: cells in the order of their first
+// modes, every fourth to a partial sum, those added in pairs.  Returns their number.
+int twin_direct_cells(double *out, const long long *idx, long nidx, const double *interp,
+                      const double *pt, const double *pcoef, const int *m, const int *k,
+                      const int *n, int L, int out_len, int K, const double *ylm, double dt,
+                      const double *h_t)
+{
+    std::vector<int> st(L), en(L);
+    twin_plan(h_t, L, dt, out_len, st.data(), en.data());
+    std::vector<std::vector<int>> cells;
+    for (int q = 0; q < K; q++) {
+        size_t c = 0;
+        while (c < cells.size() && (m[cells[c][0]] != m[q] || k[cells[c][0]] != k[q] ||
+                                    n[cells[c][0]] != n[q]))
+            c++;
+        if (c == cells.size()) cells.emplace_back();
+        cells[c].push_back(q);
+    }
+    const long nb = (long)L * 2 * K;
+    for (long q = 0; q < nidx; q++) {
+        SampleState ss;
+        const int j = twin_sample(h_t, pt, pcoef, L, dt, st, en, (int)idx[q], ss);
+        double re[4] = {}, im[4] = {};
+        for (size_t c = 0; j >= 0 && c < cells.size(); c++) {
+            const int lead = cells[c][0];
+            double v[4][4] = {};
+            for (int mode : cells[c])
+                for (int p = 0; p < 4; p++) {
+                    const double *ip = interp + p * nb + (long)j * 2 * K;
+                    cell_coef_add(ip[mode], ip[K + mode], ylm[2 * mode], ylm[2 * mode + 1],
+                                  ylm[2 * (K + mode)], ylm[2 * (K + mode) + 1], m[lead] != 0, v[p]);
+                }
+            cell_term_fp64<false>(v, m[lead], k[lead], n[lead], ss.x, ss.Pp, ss.Pt, ss.Pr, re[c % 4],
+                                  im[c % 4]);
+        }
+        out[2 * q] = (re[0] + re[1]) + (re[2] + re[3]);
+        out[2 * q + 1] = (im[0] + im[1]) + (im[2] + im[3]);
+    }
+    return (int)cells.size();
+}
+
+// Direct FP64 mode sum at chosen samples with the reference's per-mode code.
 int twin_direct_samples(double *out, const long long *idx, long nidx, const double *interp,
                         const double *pt, const double *pcoef, const int *m, const int *k,
                         const int *n, int L, int out_len, int K, const double *ylm, double dt,
@@ -116,26 +176,12 @@ int twin_direct_samples(double *out, const long long *idx, long nidx, const doub
 {
     std::vector<int> st(L), en(L);
     twin_plan(h_t, L, dt, out_len, st.data(), en.data());
-    const long np = (long)(L - 1) * 3;
     const long nb = (long)L * 2 * K;
     for (long q = 0; q < nidx; q++) {
-        const int i = (int)idx[q];
-        int j = -1;
-        for (int jj = 0; jj < L - 1; jj++)
-            if (i >= st[jj] && i < en[jj]) {
-                j = jj;
-                break;
-            }
+        SampleState ss;
+        const int j = twin_sample(h_t, pt, pcoef, L, dt, st, en, (int)idx[q], ss);
         double w_re = 0.0, w_im = 0.0;
         if (j >= 0) {
-            double rp[8], rt[8], rr[8];
-            for (int c = 0; c < 8; c++) {
-                rp[c] = pcoef[c * np + (long)j * 3 + 0];
-                rt[c] = pcoef[c * np + (long)j * 3 + 1];
-                rr[c] = pcoef[c * np + (long)j * 3 + 2];
-            }
-            SampleState ss;
-            sample_state(dt, i, h_t[j], pt[j], pt[j + 1] - pt[j], rp, rt, rr, ss);
             double tr_re = 0.0, tr_im = 0.0;
             for (int mode = 0; mode < K; mode++) {
                 if (mode > 0 && mode % 5000 == 0) {
@@ -179,7 +225,7 @@ void twin_sincos_cw(const double *x, double *s, double *c, int *ok, long n)
     for (long i = 0; i < n; i++) ok[i] = sincos_cw(x[i], s[i], c[i]) ? 1 : 0;
 }
 
-// The frequency-domain sum with the kernel's per-item and per-bin routines,
+// The frequency-domain sum with the reference's per-item and per-bin routines,
 // in the CPU branch's loop order (modes, segments, bins, roots) with plain
 // sequential adds: bit-comparable with the oracle.
 int twin_fd_waveform(double *wave, const double *interp, const double *phase_t,
@@ -255,7 +301,7 @@ int twin_interp2d(double *z, const double *tx, int nx, const double *ty, int ny,
     return 0;
 }
 
-// The AAK sum with the kernel's plan and per-sample routine, segment by
+// The AAK sum with the reference's plan and per-sample routine, segment by
 // segment in the CPU branch's order.
 int twin_aak_waveform(double *wave, const double *interp, double M, double S, double mu,
                       double qS, double phiS, double qK, double phiK, double dist, int nmodes,
@@ -475,7 +521,7 @@ int twin_fd_waveform_fast(double *wave, const double *interp, const double *phas
     return 0;
 }
 
-// fd_amp, and fd_bin's form of the same factor
+// fd_amp, and the reference's form of the same factor
 void twin_fd_amp(const double *fdot, const double *fddot, long n, double *fast, double *ref)
 {
     const FdSpaConst kc = fd_spa_const();

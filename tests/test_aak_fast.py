@@ -44,7 +44,7 @@ def test_bessel5_degenerate(twin):
     fast, ref = np.zeros((6, 5)), np.zeros((6, 5))
     twin.twin_aak_bessel5.argtypes = [P, P, ctypes.c_long, P, P]
     twin.twin_aak_bessel5(_p(order), _p(x), 6, _p(fast), _p(ref))
-    np.testing.assert_array_equal(fast[:5], ref[:5])
+    np.testing.assert_array_equal(fast, ref)
 
 
 @pytest.mark.parametrize("mich", [False, True])

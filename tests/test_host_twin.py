@@ -134,6 +134,7 @@ def test_twin_plan_matches_find_start_inds(tw, out_delta):
 
 
 def test_twin_direct_fp64_vs_oracle(tw):
+    """The reference's mode term (twin_reference.hpp), mode by mode."""
     from fastemriwaveforms_amd import synthetic
     inp = synthetic.make_workload("cpu0")
     interp, pcoef = oracle_coefficients(inp)
@@ -145,6 +146,32 @@ def test_twin_direct_fp64_vs_oracle(tw):
                            _p(k), _p(n), inp.L, inp.num_pts, inp.K, _p(yl), inp.dt, _p(inp.t))
     ref = oracle_waveform(inp, idx)
     assert oracle.rel_l2(out.view(np.complex128), ref) < 1e-14
+
+
+@pytest.mark.parametrize("kind", ["cpu0", "shuffled", "polar"])
+def test_twin_direct_cells_vs_oracle(tw, kind):
+    """The kernels' sum over cells (cell_coef_add, cell_term_fp64, every fourth cell,
+    the four sums in pairs) at samples of a workload: the bar of the GPU comparison
+    (phases are identical; ~20 rounded operations per mode)."""
+    from fastemriwaveforms_amd import synthetic
+    if kind == "polar":
+        inp = synthetic.make_input(0.05, 10.0, 30, "k1_20", 400, 3, phases="dopr")
+    else:
+        inp = synthetic.make_workload("cpu0")
+    order = np.random.default_rng(2).permutation(inp.K) if kind == "shuffled" else np.arange(inp.K)
+    interp, pcoef = oracle_coefficients(inp)
+    idx = spread_indices(inp.num_pts, count=300)
+    out = np.zeros(2 * len(idx))
+    i32 = lambda a: np.ascontiguousarray(a[order], np.int32)
+    m, k, n = i32(inp.m), i32(inp.k), i32(inp.n)
+    cols = np.concatenate([order, inp.K + order])
+    it = np.ascontiguousarray(interp.reshape(4, inp.L, 2 * inp.K)[:, :, cols])
+    yl = np.ascontiguousarray(inp.ylms[cols])
+    tw.twin_direct_cells.argtypes = tw.twin_direct_samples.argtypes
+    cells = tw.twin_direct_cells(_p(out), _p(idx), len(idx), _p(it), _p(inp.t), _p(pcoef), _p(m),
+                                 _p(k), _p(n), inp.L, inp.num_pts, inp.K, _p(yl), inp.dt, _p(inp.t))
+    assert cells == len(np.unique(np.stack([m, k, n]), axis=1).T)
+    assert oracle.rel_l2(out.view(np.complex128), oracle_waveform(inp, idx)) < 1e-12
 
 
 def test_twin_sincos_turns(tw):

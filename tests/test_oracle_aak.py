@@ -1,6 +1,6 @@
 """Pins of the AAK oracle (oracle/few_oracle_aak.c, the CPU branch of
-gpuAAK.cu's get_waveform) and of the kernel's per-sample code against it
-(host twin).
+gpuAAK.cu's get_waveform) and of the host twin's restatement of its sample against
+it (the kernel's own form is held against the oracle in test_aak_fast.py).
 
 * the Numerical Recipes Bessel functions against scipy's jv, bounded per
   order by the routines' own accuracy (Miller's recurrence started at
@@ -174,8 +174,8 @@ def test_twin_bessel_bitwise(twin):
 
 
 def test_twin_aak_bitwise(twin):
-    """The kernel's per-sample routine, run on the host over the oracle's plan,
-    equals the oracle bit for bit (host libm on both sides)."""
+    """The reference's sample and plan (twin_reference.hpp) equal the oracle bit for
+    bit (host libm on both sides)."""
     twin.twin_aak_waveform.argtypes = [P, P] + [ctypes.c_double] * 8 + [
         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_double, P]
     for mich in (False, True):

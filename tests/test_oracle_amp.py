@@ -1,6 +1,6 @@
 """Pins of the amplitude-interpolation oracle (oracle/few_oracle_amp.c, the
 CPU branch of interp2D, src/few/cutils/AmpInterp2D.cu:1-208) and of the
-kernel's per-point basis / per-set sum against it (host twin).
+kernel's interval, weights and per-set sum against it (host twin).
 
 FITPACK's bispev (scipy.interpolate.bisplev) evaluates the same
 tensor-product B-spline with the same routines (fpbspl, fpbisp): the oracle

@@ -1,6 +1,7 @@
 """Pins of the frequency-domain oracle (oracle/few_oracle_fd.c, the CPU branch
 of get_waveform_generic_fd, src/few/cutils/interpolate.cu:1142-1563) and of
-the kernel's per-bin code against it (host twin).
+the host twin's restatement of its bin against it (the kernels' own form is held
+against that in test_fd_fast.py).
 
 * SPAFunc against scipy's modified Bessel function: the routine equals
   -i sqrt(x) e^{-ix} K_1/3(-ix) (principal branches) up to the truncation of
@@ -9,8 +10,8 @@ the kernel's per-bin code against it (host twin).
 * the whole sum, as test_fd.py checks the reference (tests/test_fd.py:70-140):
   the overlap of h+ with the FFT of the time-domain waveform's real part, and
   its absolute scale: |h+|^2 = dt^2 |FFT|^2 band by band;
-* the kernel's item/bin routines, run on the host in the oracle's loop order,
-  equal the oracle bit for bit.
+* the reference's item and bin (twin_reference.hpp), run on the host in the
+  oracle's loop order, equal the oracle bit for bit.
 """
 
 import ctypes
@@ -149,8 +150,9 @@ def tw(twin):
 @pytest.mark.parametrize("include_minus_m,separate_modes", [(True, False), (False, False),
                                                             (True, True)])
 def test_twin_fd_bitwise(tw, include_minus_m, separate_modes):
-    """The kernel's fd_load_item / fd_bin, looped in the CPU branch's order,
-    equal the oracle bit for bit (host libm on both sides)."""
+    """The reference's item and bin (twin_reference.hpp, which the kernels' form is
+    held against in test_fd_fast.py), looped in the CPU branch's order, equal the
+    oracle bit for bit (host libm on both sides)."""
     inp = _small(T=0.02, L=25, K=10, seed=3)
     freq = oracle.fd_frequency_grid(inp.num_pts, 1 - inp.num_pts % 2, inp.dt)
     ref, (start, end, zero) = oracle_fd(inp, freq, include_minus_m=include_minus_m,
