@@ -599,10 +599,9 @@ __global__ __launch_bounds__(FD_SCAN_BLOCK) void fd_scan3_kernel(const long *loc
 
 // separate_modes: persistent walk over the flattened bins: workgroup b owns a
 // contiguous range; each thread strides through it, reloading the item only
-// when its next bin belongs to another (mode, segment).  Capped at 256 registers, two
-// waves per SIMD: the per-bin chains of FP64 libm calls are latency-bound,
-// and a second wave hides more of that than the few spills it costs
-// (measured on full1-sized FD sums: 133 ms against 164 ms at one wave).
+// when its next bin belongs to another (mode, segment).  Two waves per SIMD (197
+// registers): 60 modes of one year 0.98 ms (one wave 1.56, three with 36 registers
+// spilled 1.02, four 1.65).
 __global__ __launch_bounds__(FD_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fd_sum_kernel(FdArgs a, long nitems)
 {
@@ -1147,11 +1146,10 @@ int launch_fd_sum(FdArgs a, void *workspace, size_t workspace_bytes, hipStream_t
     int dev = 0, ncu = 256;
     FEW_HIP(hipGetDevice(&dev));
     FEW_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    // 64 workgroups per CU, each a contiguous bin range: short ranges balance
-    // the uneven per-bin cost (roots in or out of the segment, the SPA branch)
-    // better than a few long ones (full1-sized FD sum: 124 ms at 64 per CU,
-    // 133 ms at 8, 138 ms at 2)
-    hipLaunchKernelGGL(fd_sum_kernel, dim3((unsigned)(ncu * 64)), dim3(FD_THREADS), 0, stream, a,
+    // 8 workgroups per CU, each a contiguous bin range: 300 modes of 0.1 yr 0.72 ms,
+    // 6 modes of 0.02 yr 25 us (64 per CU 0.85 ms and 99 us: short ranges form their
+    // first item for few bins)
+    hipLaunchKernelGGL(fd_sum_kernel, dim3((unsigned)(ncu * 8)), dim3(FD_THREADS), 0, stream, a,
                        nitems);
     FEW_HIP(hipGetLastError());
     return FEW_OK;
