@@ -482,9 +482,13 @@ int launch_plan(const PlanArgs &p, hipStream_t stream)
 // samples), 9468 samples 7.9 / 9.5 / 10.5 / 12.6 us (7.7 / 8.0 / 8.0 / 8.6).
 static bool direct_few(long out_len, int K) { return K <= DIRECT_FEW && out_len >= 4096L * K; }
 
-// Otherwise, below 2^17 samples the four-sample tiles are too few to fill the chip:
-// 63,116 samples of the full set take 128 us with one sample per lane and 183 us
-// with four, 315,582 samples of 500 modes 193 us with four and 217 us with one.
+// Otherwise, below 2^17 samples the four-sample tiles are too few to fill the chip.
+// One against four samples per lane, us (plan and cell index included):
+//                     16,000     64,000     100,000    131,072    300,000 samples
+//   20 modes          10 / 12    13 / 14    16 / 14    18 / 17    28 / 23
+//   500 modes         46 / 64    72 / 94    97 / 93    118 / 124  225 / 194
+//   3843 modes        117 / 143  170 / 202  224 / 204  278 / 261  508 / 401
+// (the means of 30 and 120 knots, which change little).
 int direct_tile(long out_len, int K)
 {
     if (direct_few(out_len, K)) return DIRECT_FEW_TILE;

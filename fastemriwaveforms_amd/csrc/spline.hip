@@ -29,10 +29,10 @@ namespace few {
 #define SPLINE_MAX_GROUPS 4
 #define SPLINE_PF 8  // prefetch distance (steps) of the sequential sweeps
 // LDS path: (2 * 32 + 6) * L doubles per 32-system block, 290 knots in 160 KiB.
-// Above 146 knots a CU holds one block instead of two, which still wins where
-// there is more than a block per CU: 7686 systems of 151 / 200 knots take 62 /
-// 80 us (134 / 175 us with a lane per system and its scratch in HBM), 30000 of
-// 290 knots 397 us (534).
+// A CU holds one block at any length: a lane of the kernel takes 364 registers, those
+// of the per-lane path of singular systems included, so a SIMD has one wave.  7686
+// systems of 151 / 200 / 290 knots take 55 / 71 / 100 us (134 / 175 us at 151 / 200
+// with a lane per system and its scratch in HBM), 30000 of 290 knots 386 us (534).
 #define SPLINE_SHARED_MAX_L 290
 // Knots from which the chains of a block follow each other (below).  With fewer the
 // counters cost more than the overlap gives: 7686 systems of 8 / 10 / 12 knots 8.5 /
@@ -568,7 +568,7 @@ __device__ __forceinline__ int spline_peek(int *c)
 // Below SPLINE_FOLLOW knots the same steps go one after the other, with divisions and
 // the coefficients on all four waves.
 // What bounds it: the latency of those chains, one dependent FP64 operation after
-// another.  7686 systems of 120 knots: 45 us; 30000 of 290 knots: 397 us (57
+// another.  7686 systems of 120 knots: 45 us; 30000 of 290 knots: 386 us (57
 // and 485 us with the chains, 18 us for the elimination and 21 us for the sweeps,
 // and the coefficients one after the other, and a division per step of the back
 // substitution).

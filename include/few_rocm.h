@@ -155,10 +155,11 @@ size_t few_plan_workspace_bytes(const void *plan, int init_len, int out_len, int
  * 1 = prepare (interval planning, coefficient tiles), 2 = sum (the output
  * kernel), 3 = both; stage 2 reuses what the last stage-1 call on the same
  * workspace prepared, and is refused (FEW_ERR_ARG) unless that call had the
- * same plan, precision, variant, init_len and out_len.  Adding 4 to a stage with the sum (6, 7) overwrites
- * instead of accumulating: every output sample is written (h where an
- * interval covers it, 0 after the last one), so the caller need not zero
- * d_waveform first.  Workspace:
+ * same plan, precision, variant, init_len and out_len (FP64: the modes may be
+ * others, the interval plan does not depend on them).  Adding 4 to a stage
+ * with the sum (6, 7) overwrites instead of accumulating: every output sample
+ * is written (h where an interval covers it, 0 after the last one), so the
+ * caller need not zero d_waveform first.  Workspace:
  * few_plan_workspace_bytes() bytes, caller-owned, one call in flight at a
  * time.  No host synchronisation, no allocation: capturable in a hipGraph.
  */
@@ -338,9 +339,9 @@ int few_fd_workspace_bytes(int num_teuk_modes, int num_segments, size_t *bytes);
  * delta_t is accepted and unused, as in the reference kernel.  Differences
  * from the reference, both on inputs the reference mishandles: bins outside
  * [0, data_length) are skipped before the frequency is read, and a -m bin
- * outside the array is dropped instead of written out of bounds.  Colliding
- * bins are added with FP64 atomics, so their summation order is not fixed
- * (as with the reference's atomic adds).  Stream-ordered. */
+ * outside the array is dropped instead of written out of bounds.  Every bin is
+ * summed by one thread in a fixed order: the output is the same on every run
+ * (the reference adds with atomics).  Stream-ordered. */
 int few_get_waveform_generic_fd_async(void *waveform, const double *interp_array,
                                       const double *phase_interp_t,
                                       const double *phase_interp_coeffs, const int *m,
@@ -425,8 +426,10 @@ int few_release_workspace(void);
  * forbid hipMalloc): few_get_waveform_plan_async with the same arguments
  * except the workspace, which comes from a library-owned static device
  * array of FEW_NOALLOC_SCRATCH_BYTES per GPU (held until the process ends).
- * A call whose few_plan_workspace_bytes() exceeds that size is refused with
- * FEW_ERR_LIMIT (FP64 needs ~36 B per knot; MIXED16 adds the coefficient
+ * A call whose needs exceed that size is refused with FEW_ERR_LIMIT: for FP64 the
+ * interval plan, ~36 B per knot (the index of modes sharing (m, k, n), 24 B per mode,
+ * is used where it fits beside the plan); for the others
+ * few_plan_workspace_bytes() (MIXED16 adds the coefficient
  * tiles: 5.4 MB for 120 knots and the 3843-mode set, 18 MB for 200 knots
  * and n in [-55, 55]; FACT64 its FP64 tiles, 11 MB and 32 MB).  The call allocates nothing: no hipMalloc / hipFree
  * and no allocating library routine.  Every call on one GPU shares that
