@@ -136,7 +136,6 @@ __host__ __device__ inline fcx fcx_div(fcx z, fcx w)
     return fcx_make(x, y);
 }
 
-__host__ __device__ inline fcx fcx_rdiv(double x, fcx w) { return fcx_div(fcx_make(x, 0.0), w); }
 __host__ __device__ inline double fcx_abs(fcx z) { return hypot(z.re, z.im); }
 __host__ __device__ inline double fcx_arg(fcx z) { return atan2(z.im, z.re); }
 

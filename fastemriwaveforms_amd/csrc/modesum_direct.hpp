@@ -71,7 +71,7 @@ __host__ __device__ inline void plan_interval(const double *h_t, int j, int used
 }
 
 struct SampleState {
-    double x, x2, x3;     // x = t - h_t[j] and its powers (amplitude cubic)
+    double x;             // x = t - h_t[j] (amplitude cubic)
     double Pp, Pt, Pr;    // Phi_phi, Phi_theta, Phi_r at t
 };
 
@@ -105,8 +105,6 @@ __host__ __device__ inline void sample_state(double dt, int i, double h_t, doubl
 #pragma clang fp contract(off)
     const double t = dt * (double)i;
     st.x = t - h_t;
-    st.x2 = st.x * st.x;
-    st.x3 = st.x * st.x2;
     const double s = (t - pt) / pw;
     const double s1 = 1.0 - s;
     st.Pp = dense_phase(rp, s, s1);

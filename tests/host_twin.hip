@@ -196,7 +196,7 @@ int twin_direct_samples(double *out, const long long *idx, long nidx, const doub
                 c.yp_re = ylm[2 * mode]; c.yp_im = ylm[2 * mode + 1];
                 c.ym_re = ylm[2 * (K + mode)]; c.ym_im = ylm[2 * (K + mode) + 1];
                 c.m = m[mode]; c.k = k[mode]; c.n = n[mode];
-                mode_term_fp64(c, ss.x, ss.x2, ss.x3, ss.Pp, ss.Pt, ss.Pr, tr_re, tr_im);
+                mode_term_fp64(c, ss.x, ss.x * ss.x, ss.x * (ss.x * ss.x), ss.Pp, ss.Pt, ss.Pr, tr_re, tr_im);
             }
             w_re = w_re + tr_re;
             w_im = w_im + tr_im;

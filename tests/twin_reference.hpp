@@ -44,6 +44,8 @@ inline void mode_term_fp64(const ModeCoef &c, double x, double x2, double x3,
 // --------------------------------------------------------- frequency domain
 #pragma clang fp contract(off)
 
+inline fcx fcx_rdiv(double x, fcx w) { return fcx_div(fcx_make(x, 0.0), w); }
+
 // cube_roots (interpolate.cu:1113-1134): Cardano with the principal complex
 // cube root; xi = (-1 + sqrt(-3)) / 2 is passed in (computed once per thread).
 inline void fd_cube_roots(double a, double b, double c, double d, fcx xi,
